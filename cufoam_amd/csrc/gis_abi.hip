@@ -139,6 +139,7 @@ GIS_API int gis_create(gis_handle* out, int device) {
     if (hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, device) == hipSuccess &&
         wall_khz > 0)
         h->wall_tick = 1.0 / (1000.0 * wall_khz);
+    (void)hipDeviceGetAttribute(&h->n_cu, hipDeviceAttributeMultiprocessorCount, device);
     if (ensure_state(h) != kOK || noalloc_setup(h) != kOK) {
         if (h->st_host) (void)hipHostFree(h->st_host);
         (void)hipStreamDestroy(h->stream);
@@ -479,6 +480,7 @@ GIS_API int gis_set_schedule(gis_handle h, const gis_schedule* s) {
     if (s->spmv64 > 6 || s->spmv32 > 6 || s->fp64_direction > 1 || s->fp32_direction > 1 ||
         !coarsen_ok(s->coarsen64) || !coarsen_ok(s->coarsen32))
         return fail(h, GIS_ERR_ARG, "schedule field out of range");
+    if (s->spmv64 >= 0 || s->fp64_direction >= 0 || s->coarsen64 > 0) h->sched_pinned = true;
     if (s->spmv64 >= 0) h->sched.spmv64 = static_cast<SpmvKind>(s->spmv64);
     if (s->spmv32 >= 0) h->sched.spmv32 = static_cast<SpmvKind>(s->spmv32);
     if (s->block_iters > 0) h->sched.block_iters = s->block_iters;

@@ -189,6 +189,7 @@ struct gis_context {
     // table entries, tabled slices with one-byte masks, sliced-row slots of the others
     long long lay_slices = 0, lay_table_slices = 0, lay_table_entries = 0;
     long long lay_byte_mask_slices = 0, lay_untabled_slots = 0;
+    int lay_max_table = 0, lay_max_row = 0;     // longest offset table, longest row
     gis::DevMem dval, dvalT, dval32, dval32T;
     // symmetric storage of the SellD layout (every slice tabled): the FP64 slot
     // values of the table entries with column offset >= 0 only (dsv), and per
@@ -219,6 +220,10 @@ struct gis_context {
     gis::DevMem mstate;                         // per-column states of multi-RHS solves
     gis::KState* mstate_host = nullptr;         // pinned mirror
     gis::DevMem io2;                            // staging for multi-RHS / adjoint data
+    gis::DevMem res_mem;                        // slots and handshake of resident solves
+    int n_cu = 0;                               // compute units of the device
+    bool sched_pinned = false;                  // gis_set_schedule chose the FP64 kernels
+    bool res_unfit = false;                     // the pattern takes no resident form
 
     gis::Schedule sched;
     gis::Timer timer;
@@ -368,6 +373,22 @@ int device_solve_multi_mixed(gis_context* h, int method, int nrhs, const MultiMi
 // dL_k/dA = -lambda_k x^T on the pattern, written into LDU-shaped gradients.
 int device_sddmm_fold(gis_context* h, int nrhs, const double* Lam, const double* x,
                       double* d_diag, double* d_lower, double* d_upper);
+
+// CG and BiCG as resident launches where the system fits the chip
+// (gis_resident.hip), from the state and residual that k_setup left.  *ran =
+// false: nothing was done (no resident form, another resident solve is running,
+// or the grid could not be made resident), and the caller iterates with its own
+// launches; else the solve is over, x complete.  p, ps and qx (kResQ vectors per
+// exchanged one) are workspace.
+constexpr int kResQ = 3;
+template <typename T>
+struct Mat;
+bool resident_cg_fits(const gis_context* h);
+bool resident_bicg_fits(const gis_context* h);
+int resident_cg(gis_context* h, const Mat<double>& m, double* r, double* p, double* qx, double* x,
+                bool* ran);
+int resident_bicg(gis_context* h, const Mat<double>& m, const Mat<double>& mt, double* r,
+                  double* rs, double* p, double* ps, double* qx, double* x, bool* ran);
 
 // batched systems (gis_batch.hip); addressing is per system (local cell ids),
 // faces and coefficients concatenated system by system

@@ -416,5 +416,11 @@ int run_blocks(gis_context* h, long long max_steps, Iter&& launch_iteration,
 }
 
 int prepare_solve(gis_context* h, const SolveArgs& a, int nvec);
+// CG with the matrix m, BiCG with m and its transpose mt; the state is left on the
+// device, with a mirror in h->st_host
+int solve_cg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, double* x,
+                const double* b);
+int solve_bicg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, const Mat<double>& mt,
+                  double* x, const double* b);
 
 }  // namespace gis

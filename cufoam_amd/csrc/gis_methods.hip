@@ -692,7 +692,14 @@ int solve_richardson(gis_context* h, const SolveArgs& a, double* x, const double
 
 int solve_bicg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
     GIS_TRY(ensure_valT(h));
-    GIS_TRY(prepare_solve(h, a, 6));
+    return solve_bicg_on(h, a, mat64(h), mat64T(h), x, b);
+}
+
+}  // namespace
+
+int solve_bicg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, const Mat<double>& mt,
+                  double* x, const double* b) {
+    GIS_TRY(prepare_solve(h, a, resident_bicg_fits(h) ? 4 + 2 * kResQ : 6));
     const int N = h->N;
     double* r = h->vec.as<double>();
     double* rs = r + N;
@@ -700,9 +707,10 @@ int solve_bicg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
     double* pb1 = r + 3 * (size_t)N;
     double* ps = r + 4 * (size_t)N;
     double* q = r + 5 * (size_t)N;
-    const Mat<double> m = mat64(h);
-    const Mat<double> mt = mat64T(h);
     GIS_TRY(launch_setup(h, m, b, x, nullptr, r, rs, 1));
+    bool resident = false;   // p in pb0, p* in pb1, the exchanged q and q* from ps on
+    GIS_TRY(resident_bicg(h, m, mt, r, rs, pb0, pb1, ps, x, &resident));
+    if (resident) return kOK;
     const dim3 g = tiles_grid(N);
     GIS_SPMV_DISPATCH(h->sched.spmv64, P, {
         GIS_TRY(run_blocks(h, iteration_budget(h), [&]() -> int {
@@ -722,6 +730,8 @@ int solve_bicg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
     });
     return kOK;
 }
+
+namespace {
 
 // BiCG preconditioned by M = D (no counterpart in the reference): the BiCG
 // loop, breakdown test, stopping rule and history, with z = D^-1 r in the

@@ -760,6 +760,36 @@ int solve_multi_mixed_nr(gis_context* h, int method, const MultiMixedArgs& a, do
     return kOK;
 }
 
+// Columns solved one after another, each as a single-RHS solve (the bits of its
+// column in the SpMM solve).
+int solve_columns(gis_context* h, int method, int nrhs, bool transpose, const SolveArgs& a,
+                  double* X, const double* B, int* iters, double* norm0, double* normf,
+                  int* status) {
+    const Mat<double> mA = transpose ? mat64T(h) : mat64(h);
+    const Mat<double> mAt = transpose ? mat64(h) : mat64T(h);
+    const size_t n = (size_t)h->N;
+    int worst = kOK;
+    for (int k = 0; k < nrhs; ++k) {
+        GIS_TRY(method == 0 ? solve_cg_on(h, a, mA, X + k * n, B + k * n)
+                            : solve_bicg_on(h, a, mA, mAt, X + k * n, B + k * n));
+        GIS_TRY(read_state(h));
+        const KState& s = *h->st_host;
+        int sk = s.status;
+        if (sk == kOK && !(s.norm == s.norm)) sk = kNaN;
+        if (iters) iters[k] = s.k;
+        if (norm0) norm0[k] = s.norm0;
+        if (normf) normf[k] = s.norm;
+        if (status) status[k] = sk;
+        worst = std::max(worst, sk);
+    }
+    return worst;
+}
+
+// Columns up to which that is the faster form (one, two, three and five columns
+// against one SpMM solve: CG 2.1x, 1.3x, 1.1x, 1.0x at 64^3 and 2.3x, 1.6x, 1.3x,
+// 1.0x at 63^3 renumbered; BiCG the same within 5%; faster still below).
+constexpr int kResColumns = 3;
+
 #define GIS_NR_DISPATCH(nrhs, NRC, ...)                     \
     switch (nrhs) {                                         \
         case 1: { constexpr int NRC = 1; __VA_ARGS__; } break; \
@@ -780,6 +810,9 @@ int device_solve_multi(gis_context* h, int method, int nrhs, bool transpose, con
     if (nrhs < 1 || nrhs > kMaxRhs) return fail(h, kErrArg, "nrhs must be in 1..8");
     if (method != 0 && method != 1) return fail(h, kErrArg, "multi-RHS solves support CG and BiCG");
     GIS_TRY(ensure_valT(h));
+    // a few columns of a system that fits the chip: one resident solve each
+    if (nrhs <= kResColumns && (method == 0 ? resident_cg_fits(h) : resident_bicg_fits(h)))
+        return solve_columns(h, method, nrhs, transpose, a, X, B, iters, norm0, normf, status);
     MultiBufs mb;
     GIS_TRY(multi_prepare(h, nrhs, a, sizeof(double) * (size_t)h->N * 6 * nrhs, mb));
     int st = kOK;

@@ -506,18 +506,25 @@ int prepare_solve(gis_context* h, const SolveArgs& a, int nvec) {
 }
 
 int solve_cg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
-    GIS_TRY(prepare_solve(h, a, 4));
+    return solve_cg_on(h, a, mat64(h), x, b);
+}
+
+int solve_cg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, double* x,
+                const double* b) {
+    GIS_TRY(prepare_solve(h, a, resident_cg_fits(h) ? 2 + kResQ : 4));
     const int N = h->N;
     double* r = h->vec.as<double>();
     double* pb0 = r + N;
     double* pb1 = r + 2 * (size_t)N;
     double* q = r + 3 * (size_t)N;
     const dim3 g = tiles_grid(N);
-    const Mat<double> m = mat64(h);
     GIS_SPMV_DISPATCH(h->sched.spmv64, P, {
         hipLaunchKernelGGL((k_setup<P>), g, dim3(kWG), 0, h->stream, m, N, b, x, nullptr, r,
                            nullptr, h->st, h->red, 0);
         GIS_HIP(h, hipGetLastError());
+        bool resident = false;   // p in pb0, the exchanged q from pb1 on
+        GIS_TRY(resident_cg(h, m, r, pb0, pb1, x, &resident));
+        if (resident) return kOK;
         const bool split = h->sched.fp64_direction != 0;
         GIS_COARSEN_DISPATCH(h->sched.coarsen64, CC, {
             const dim3 gc = super_grid(N, CC);

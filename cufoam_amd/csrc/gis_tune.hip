@@ -136,7 +136,9 @@ int device_autotune(gis_context* h, int what, int iterations, int* spmv, int* di
     hipLaunchKernelGGL(k_fill_probe<double>, g1, dim3(256), 0, h->stream, N, b, 1.0);
     const Schedule saved = h->sched;
     const unsigned timer_mask = h->timer.mask;
+    const bool pinned = h->sched_pinned;
     h->timer.mask = 0;
+    h->sched_pinned = true;   // the candidates are the launch-per-stage kernels
     auto apply = [&](const Candidate& c) {
         if (fp64) {
             h->sched.spmv64 = static_cast<SpmvKind>(c.spmv);
@@ -263,6 +265,7 @@ int device_autotune(gis_context* h, int what, int iterations, int* spmv, int* di
     apply(kCandidates[0]);
     const int st = sweep();
     h->sched = saved;
+    h->sched_pinned = pinned;
     h->timer.mask = timer_mask;
     if (st != kOK) return st;
     if (best_i < 0) return fail(h, kErrState, "autotune: no candidate passed the parity gate");
@@ -282,6 +285,7 @@ int device_autotune(gis_context* h, int what, int iterations, int* spmv, int* di
 
 void pattern_schedule(gis_context* h) {
     Schedule& s = h->sched;
+    h->sched_pinned = false;
     // SellD when the offset tables cover all but a sliver of the matrix (the
     // slices without a table read int32 columns inside the same kernels; a
     // batch's padding slices are such slices)

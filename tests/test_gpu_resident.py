@@ -1,0 +1,148 @@
+"""Resident CG and BiCG (gis_resident.hip): one launch per solve where the system
+fits the chip.  Sizes where the route or a tile remainder changes: a single
+workgroup of one tile and of two, the first that exchange halos, ragged last
+tiles and slices, the largest of one tile per workgroup and the first of two,
+the first that does not fit; both slot forms; a halo too large for two tiles; rows
+with too many entries.  Every result equals the launch-per-stage kernels' (the
+schedule chosen explicitly) bit for bit, and the oracle's where that is quick."""
+import numpy as np
+import pytest
+
+from cufoam_amd import mesh
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def stages(g, f):
+    """f(g) with the schedule in force chosen explicitly: the launch-per-stage loop."""
+    g.set_schedule(spmv64=g.get_schedule()["spmv64"])
+    return f(g)
+
+
+def banded(n, width, seed):
+    """n cells on a line, each coupled to the next and to the one `width` on."""
+    rng = np.random.default_rng(seed)
+    c = np.arange(n)
+    pairs = np.concatenate([np.stack([c[:-1], c[1:]], 1), np.stack([c[:-width], c[width:]], 1)])
+    pairs = pairs[np.lexsort((pairs[:, 1], pairs[:, 0]))]
+    la, ua = pairs[:, 0].astype(np.int32), pairs[:, 1].astype(np.int32)
+    up = -(1.0 + 0.5 * rng.random(len(la)))
+    lo = up * (1.0 + 0.5 * rng.random(len(la)))
+    diag = mesh.row_abs_sum(n, la, ua, lo, up) + 0.1
+    return mesh.LduSystem(n, la, ua, diag, lo, up, rng.uniform(-1, 1, n), np.zeros(n))
+
+
+def symmetric(s):
+    return mesh.LduSystem(s.n_cells, s.lower_addr, s.upper_addr,
+                          mesh.row_abs_sum(s.n_cells, s.lower_addr, s.upper_addr, s.upper,
+                                           s.upper) + 0.1, s.upper, s.upper, s.b, s.x0)
+
+
+SIZES = [1, 3, 63, 64, 65, 1023, 1024, 1025, 2047, 2048, 2049, 3072, 4099, 65 * 1024 + 1,
+         129 * 1024 - 3, 256 * 1024, 256 * 1024 + 1, 512 * 1024, 512 * 1024 + 1]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_resident_equals_stages(gpu, n, method):
+    """Column offsets 1 and a large one: tables up to the remainders, far halos."""
+    if n < 4:
+        s = mesh.random_ldu(n, n, seed=n) if n > 1 else mesh.laplacian(1)
+    else:
+        s = banded(n, max(2, min(3001, n // 3)), seed=n)
+    if method == "CG":
+        s = symmetric(s)
+    gpu.set_system(s)
+
+    def run(g):
+        return g.solve(method, s.b, s.x0, error=1e-9, max_steps=40)
+    x, hist, st = run(gpu)
+    x1, hist1, st1 = stages(gpu, run)
+    assert st == st1
+    np.testing.assert_array_equal(hist, hist1)
+    np.testing.assert_array_equal(x, x1)
+    if n <= 5000:
+        ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, 1e-9, 40)
+        np.testing.assert_array_equal(hist, ref.hist)
+        np.testing.assert_array_equal(x, ref.x)
+
+
+@pytest.mark.parametrize("n_cells,n_faces", [(900, 2500), (40000, 110000), (300000, 800000)])
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_scattered_halos_and_long_rows(gpu, n_cells, n_faces, method):
+    """Columns all over the vector: int32 slots, rows past 8 entries (not resident)."""
+    s = mesh.random_ldu(n_cells, n_faces, seed=5, symmetric=method == "CG")
+    gpu.set_system(s)
+
+    def run(g):
+        return g.solve(method, s.b, s.x0, error=1e-9, max_steps=25)
+    x, hist, _ = run(gpu)
+    x1, hist1, _ = stages(gpu, run)
+    np.testing.assert_array_equal(hist, hist1)
+    np.testing.assert_array_equal(x, x1)
+
+
+@pytest.mark.parametrize("n", [12, 40, 70])
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_random_numbering(gpu, n, method):
+    """Every neighbour in another workgroup; at 70^3 the halo of two tiles does not
+    fit and the launch gives up before it starts."""
+    s = mesh.laplacian(n, seed=3, shift=1e-2, symmetric=method == "CG")
+    s = mesh.renumber(s, np.random.default_rng(1).permutation(s.n_cells))
+    gpu.set_system(s)
+
+    def run(g):
+        return g.solve(method, s.b, s.x0, error=1e-6, max_steps=60)
+    for _ in range(2):
+        x, hist, _ = run(gpu)
+    x1, hist1, _ = stages(gpu, run)
+    np.testing.assert_array_equal(hist, hist1)
+    np.testing.assert_array_equal(x, x1)
+
+
+@pytest.mark.parametrize("n", [5, 14])
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_chunks_continue(gpu, n, method):
+    """More iterations than one launch makes: the next one goes on where it stopped."""
+    s = mesh.laplacian(n, seed=9, shift=1e-3, symmetric=method == "CG")
+    gpu.set_system(s)
+    x, hist, _ = gpu.solve(method, s.b, s.x0, error=-1.0, max_steps=4100)
+    ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, -1.0, 4100)
+    np.testing.assert_array_equal(hist, ref.hist)
+    np.testing.assert_array_equal(x, ref.x)
+
+
+def test_columns_and_transpose(gpu):
+    """Few right-hand sides of a system that fits: the SpMM solve's bits."""
+    s = mesh.laplacian(20, seed=4, shift=0.1, symmetric=False)
+    gpu.set_system(s)
+    B = np.random.default_rng(2).uniform(-1, 1, (3, s.n_cells))
+    for transpose in (False, True):
+        a = gpu.solve_multi("BiCG", B, None, error=1e-8, max_steps=300, transpose=transpose)
+        b = stages(gpu, lambda g: g.solve_multi("BiCG", B, None, error=1e-8, max_steps=300,
+                                                transpose=transpose))
+        gpu.set_system(s)
+        for u, v in zip(a, b):
+            np.testing.assert_array_equal(u, v)
+
+
+def test_infinite_and_nan_inputs(gpu):
+    """The stop rules' answers to infinities and NaN, and to a zero right-hand side."""
+    s = mesh.laplacian(13, seed=6, shift=1e-2)
+    for what in (np.inf, np.nan, 0.0):
+        b = s.b.copy()
+        if what == 0.0:
+            b[:] = 0.0
+        else:
+            b[700] = what
+        for method in ("CG", "BiCG"):
+            gpu.set_system(s)
+
+            def run(g):
+                return g.solve(method, b, s.x0, error=1e-9, max_steps=6)
+            x, hist, st = run(gpu)
+            x1, hist1, st1 = stages(gpu, run)
+            assert st == st1
+            np.testing.assert_array_equal(hist, hist1)
+            np.testing.assert_array_equal(x, x1)
