@@ -143,6 +143,11 @@ struct AmgData {
     std::vector<int> dic_ptr_f, dic_ptr_b;   // level offsets (host: launch sizes)
     DevMem dic_cells_f, dic_cells_b, dic_rd;
     int dic_kind = 0;             // the factor in dic_rd: 4 DIC, 5 DILU
+    DevMem dic_y;                 // between the sweeps: the forward sweep's result
+    // single-launch sweeps: the bricks' order and the box's strides (0: consecutive rows)
+    bool sweep_ready = false;
+    DevMem sweep_order;
+    int sweep_sx = 0, sweep_sy = 0, sweep_blocks = 0;
     void clear();
     ~AmgData();
 };
@@ -160,6 +165,7 @@ struct gis_context {
     int M = 0;
     long long nnz = 0;
     bool has_pattern = false;
+    bool upper_tri = false;     // lowerAddr < upperAddr on every face
     bool has_values = false;
     bool has_val32 = false;
     bool has_valT = false;
@@ -338,6 +344,7 @@ constexpr int kMethodPbicgDilu = 14;
 // or 5 (DILU), and z = M^-1 r by the level-scheduled sweeps with the forward
 // sweep's coefficients cf and the backward sweep's cb
 int ilu_prepare(gis_context* h, int kind);
+int ilu_begin(gis_context* h);   // before a solve's first application
 int ilu_apply(gis_context* h, const double* r, double* z, const double* cf, const double* cb);
 // Preconditioned CG (gis_amg.hip), as device_solve methods kMethodPcg0 + pc.
 int solve_pcg(gis_context* h, const SolveArgs& a, int pc, double* x, const double* b);

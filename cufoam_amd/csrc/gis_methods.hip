@@ -790,6 +790,7 @@ int solve_pbicg_dilu(gis_context* h, const SolveArgs& a, double* x, const double
     const Mat<double> mt = mat64T(h);
     GIS_TRY(launch_setup(h, m, b, x, nullptr, r, rs, 1));
     const dim3 g = tiles_grid(N);
+    GIS_TRY(ilu_begin(h));
     GIS_TRY(ilu_apply(h, r, z, lo, up));
     GIS_TRY(ilu_apply(h, rs, zs, up, lo));
     hipLaunchKernelGGL(k_pbicg_rz<1>, g, dim3(kWG), 0, h->stream, N, z, rs, h->st, h->red);

@@ -38,6 +38,7 @@ __global__ __launch_bounds__(kBlk) void k_count(int N, int M, const int* __restr
         atomicOr(err, 1);
         return;
     }
+    if (l >= u) atomicOr(err, 4);   // allowed, but the DIC/DILU sweeps then go level by level
     atomicAdd(&own_cnt[l], 1);
     atomicAdd(&nbr_cnt[u], 1);
     if (lp != l) first_own[l] = f;
@@ -592,6 +593,7 @@ int build_pattern(gis_context* h, int N, int M, const int* d_la, const int* d_ua
         return fail(h, kErrArg,
                     "face addressing invalid: need 0 <= lowerAddr, upperAddr < n_cells and "
                     "lowerAddr sorted ascending");
+    h->upper_tri = !(herr & 4);
     if (herr & 2)
         return fail(h, kErrArg, "interface entries need 0 <= row, col < n_cells and row != col");
     hipLaunchKernelGGL(k_fill_diag, grid_for(N), dim3(kBlk), 0, h->stream, N, M,
