@@ -696,25 +696,30 @@ __device__ __forceinline__ void tile_sell_c(const int* __restrict__ soff,
 // through a select.  The gather addresses therefore depend only on the
 // (scalar) offset table, not on the mask: values, masks and gathers of a batch
 // are all in flight together, one memory round trip per batch.
-template <typename T, class XOp>
+//
+// B: slots per batch.  FP32 kernels take 7 where no table is longer (the 7-point
+// stencil): with 8 the last slot of every batch is read and gathered a second
+// time (mixed CG at 256^3 191.3 -> 185.4 us per iteration, at 160^3 59.6 -> 58.6; FP64
+// CG unchanged, 366.9).
+template <typename T, int B, class XOp>
 __device__ __forceinline__ T sell_row_d(const int* __restrict__ offs, unsigned mask,
                                         const T* __restrict__ dval, int a, int len, int lane,
                                         int row, int last, XOp&& xop) {
     T acc = T(0);
-    for (int j = 0; j < len; j += 8) {
-        T v[8], xv[8];
+    for (int j = 0; j < len; j += B) {
+        T v[B], xv[B];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             const int k = min(j + u, len - 1);
             v[u] = __builtin_nontemporal_load(dval + a + k * kSlice + lane);
         }
-        int o[8];
+        int o[B];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) o[u] = offs[min(j + u, len - 1)];
+        for (int u = 0; u < B; ++u) o[u] = offs[min(j + u, len - 1)];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) xv[u] = xop(min(max(row + o[u], 0), last));
+        for (int u = 0; u < B; ++u) xv[u] = xop(min(max(row + o[u], 0), last));
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             const bool on = (mask >> (j + u)) & 1u;
             const T t = acc + v[u] * xv[u];
             acc = on ? t : acc;
@@ -724,7 +729,7 @@ __device__ __forceinline__ T sell_row_d(const int* __restrict__ offs, unsigned m
 }
 
 // Two offset-table slices per lane at a time (their loads in flight together).
-template <typename T, class XOp>
+template <typename T, int B, class XOp>
 __device__ __forceinline__ void sell_row2_d(const int* __restrict__ offs0, unsigned m0, int a0,
                                             int len0, int row0,
                                             const int* __restrict__ offs1, unsigned m1, int a1,
@@ -733,27 +738,27 @@ __device__ __forceinline__ void sell_row2_d(const int* __restrict__ offs0, unsig
                                             T& y0, T& y1) {
     T acc0 = T(0), acc1 = T(0);
     const int len = len0 > len1 ? len0 : len1;
-    for (int j = 0; j < len; j += 8) {
-        T v0[8], v1[8], x0[8], x1[8];
+    for (int j = 0; j < len; j += B) {
+        T v0[B], v1[B], x0[B], x1[B];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             const int k0 = min(j + u, len0 - 1), k1 = min(j + u, len1 - 1);
             v0[u] = __builtin_nontemporal_load(dval + a0 + k0 * kSlice + lane);
             v1[u] = __builtin_nontemporal_load(dval + a1 + k1 * kSlice + lane);
         }
-        int o0[8], o1[8];
+        int o0[B], o1[B];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             o0[u] = offs0[min(j + u, len0 - 1)];
             o1[u] = offs1[min(j + u, len1 - 1)];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             x0[u] = xop(min(max(row0 + o0[u], 0), last));
             x1[u] = xop(min(max(row1 + o1[u], 0), last));
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < B; ++u) {
             const bool on0 = (m0 >> (j + u)) & 1u, on1 = (m1 >> (j + u)) & 1u;
             const T t0 = acc0 + v0[u] * x0[u];
             const T t1 = acc1 + v1[u] * x1[u];
@@ -783,7 +788,7 @@ __device__ __forceinline__ unsigned row_mask(const unsigned* __restrict__ dmask,
     return m;
 }
 
-template <typename T, class XOp>
+template <typename T, int B, class XOp>
 __device__ __forceinline__ void tile_sell_d(const int* __restrict__ soff,
                                             const int* __restrict__ scol,
                                             const T* __restrict__ sval,
@@ -815,7 +820,7 @@ __device__ __forceinline__ void tile_sell_d(const int* __restrict__ soff,
         if (u0 > 0 && u1 > 0) {
             const unsigned m0 = row_mask(dmask, dmask8, u0, r0, N);
             const unsigned m1 = row_mask(dmask, dmask8, u1, r1, N);
-            sell_row2_d<T>(doffs + o0, m0, o0 * kSlice, u0, r0, doffs + o1, m1, o1 * kSlice,
+            sell_row2_d<T, B>(doffs + o0, m0, o0 * kSlice, u0, r0, doffs + o1, m1, o1 * kSlice,
                            u1, r1, N - 1, dval, lane, xop, y0, y1);
         } else {
 #pragma unroll
@@ -826,7 +831,7 @@ __device__ __forceinline__ void tile_sell_d(const int* __restrict__ soff,
                 T y;
                 if (up > 0) {
                     const unsigned mp = row_mask(dmask, dmask8, up, rp, N);
-                    y = sell_row_d<T>(doffs + op, mp, dval, op * kSlice, up, lane, rp, N - 1,
+                    y = sell_row_d<T, B>(doffs + op, mp, dval, op * kSlice, up, lane, rp, N - 1,
                                       xop);
                 } else {
                     const int a = soff[sp];

@@ -59,7 +59,8 @@ struct SellC {
 
 // Sliced rows with per-slice column-offset tables and row masks, two slices at
 // a time (no column index per slot).
-struct SellD {
+template <int B>
+struct SellDB {
     template <typename T>
     struct Shared {};
     template <typename T, class XOp>
@@ -72,10 +73,12 @@ struct SellD {
                 return;
             }
         }
-        tile_sell_d<T>(m.soff, m.scol, m.sval, m.ooff, m.doffs, m.dmask, m.dmask8, m.dval, N,
-                       row0, xop, y);
+        tile_sell_d<T, B>(m.soff, m.scol, m.sval, m.ooff, m.doffs, m.dmask, m.dmask8, m.dval, N,
+                          row0, xop, y);
     }
 };
+using SellD = SellDB<8>;
+using SellD7 = SellDB<7>;   // FP32, no table longer than 7
 
 // Sliced rows, two slices per lane at a time (more loads in flight per wave).
 struct Sell2 {
@@ -157,8 +160,8 @@ __device__ __forceinline__ int xcd_tile(int i, int G) {
 }
 
 // Row range of a workgroup tile.  TileRows(N): tile = workgroup index (best for
-// the SpMV-carrying kernels, measured); StreamRows(N): XCD-contiguous tiles
-// (best for the pure streaming update kernels, measured).
+// the SpMV-carrying kernels and the updates that follow them, measured);
+// StreamRows(N): XCD-contiguous tiles.
 struct TileRows {
     int tile, row0, nrows, i0;   // i0: first of this thread's kLeaf rows
     __device__ TileRows(int N) : TileRows(N, (int)blockIdx.x) {}

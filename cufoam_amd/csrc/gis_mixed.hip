@@ -256,13 +256,19 @@ __global__ __launch_bounds__(kWG) void k_mx1s(Mat<float> m, int N, const float* 
     tr.end(red, st, shr, [&](const double (&v)[1]) { finish_alpha(st, v[0]); });
 }
 
+// Rows from which k_mx2's tiles are XCD-contiguous; below, k_mx1's order, in which
+// the vectors still cached are met first (mixed CG per iteration, XCD-contiguous /
+// k_mx1's order: 160^3 58.7 / 57.9 us, 180^3 77.0 / 76.5, 200^3 102.8 / 102.8, 224^3
+// 134.9 / 136.3, 256^3 182.6 / 185.0).
+constexpr int kMx2Stream = 1 << 23;
+
 template <int C>
 __global__ __launch_bounds__(kWG) void k_mx2(int N, float* __restrict__ r,
                                              const float* __restrict__ q, KState* st,
                                              RedWs red) {
     if (st->done || (st->flag & F_UPD)) return;
     __shared__ RedShared shr;
-    const SuperTile<C> sup(N, true);
+    const SuperTile<C> sup(N, N >= kMx2Stream);
     const float af = (float)st->alpha;
     double leaf[C][1];
     float rv[C][4];
@@ -458,6 +464,8 @@ int device_solve_mixed(gis_context* h, const MixedArgs& a, double* x, const doub
     GIS_SPMV_DISPATCH(h->sched.spmv32, P32, {
         GIS_SPMV_DISPATCH(h->sched.spmv64, P64, {
             const bool split = h->sched.fp32_direction != 0;
+            constexpr bool selld = std::is_same<P32, SellD>::value;
+            const bool seven = selld && h->lay_max_table <= 7;
             GIS_COARSEN_DISPATCH(h->sched.coarsen32, CC, {
                 const dim3 gc = super_grid(N, CC);
                 GIS_TRY(run_blocks(h, max_groups, [&]() -> int {
@@ -473,8 +481,12 @@ int device_solve_mixed(gis_context* h, const MixedArgs& a, double* x, const doub
                                            N, pb0, pb1, q, h->st, h->red);
                     } else {
                         GIS_TRY(timer_begin(h, 0));
-                        hipLaunchKernelGGL((k_mx1<P32, CC>), gc, dim3(kWG), 0, h->stream, m32, N,
-                                           r32, pb0, pb1, xc, q, h->st, h->red);
+                        const auto mx1 = [&](auto k) {
+                            hipLaunchKernelGGL(k, gc, dim3(kWG), 0, h->stream, m32, N, r32, pb0,
+                                               pb1, xc, q, h->st, h->red);
+                        };
+                        if constexpr (selld) seven ? mx1(k_mx1<SellD7, CC>) : mx1(k_mx1<SellD, CC>);
+                        else mx1(k_mx1<P32, CC>);
                     }
                     GIS_TRY(timer_end(h));
                     GIS_TRY(timer_begin(h, 1));
