@@ -214,7 +214,7 @@ __global__ __launch_bounds__(kWG) void k_bcg_flush(int N, double* __restrict__ x
     const SysTile s(bv, t.tile);
     const KState* st = &bv.st[s.sys];
     const int k = st->k;
-    if (k < 1) return;
+    if (k < 1 || st->flag) return;   // flag: a resident solve's x is complete
     const double alpha = st->alpha;
     const double* p = (k & 1) ? pb1 : pb0;
     double xv[4], pv[4];
@@ -252,6 +252,7 @@ int batch_set_pattern(gis_context* h, int S, const int* n_cells, const int* n_fa
     if (B.graph_exec) (void)hipGraphExecDestroy(B.graph_exec);
     B.graph_exec = nullptr;
     h->n_cpl = 0;   // the stacked systems carry no interface entries
+    B.res_first.clear();
     B.S = S;
     B.n.assign(n_cells, n_cells + S);
     B.m.assign(n_faces, n_faces + S);
@@ -452,14 +453,17 @@ int batch_solve(gis_context* h, double* x_packed, const double* b_packed, bool d
     const int S = B.S;
     const int N = h->N;   // padded rows
     const size_t n = (size_t)N, packed = (size_t)B.pack_off[S];
-    GIS_HIP(h, h->vec.ensure(sizeof(double) * n * 6 + sizeof(double) * packed * 2));
+    const bool resident = resident_batch_fits(h);
+    GIS_HIP(h, h->vec.ensure(sizeof(double) * n * (resident ? 7 : 6) +
+                             sizeof(double) * packed * 2));
     double* x = h->vec.as<double>();
     double* b = x + n;
     double* r = b + n;
     double* pb0 = r + n;
     double* pb1 = pb0 + n;
     double* q = pb1 + n;
-    double* stage = q + n;   // packed staging (2 * packed)
+    // packed staging (2 * packed), after the third exchanged vector of a resident solve
+    double* stage = q + (resident ? 2 : 1) * n;
     const hipMemcpyKind kin = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     const hipMemcpyKind kout = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     GIS_HIP(h, hipMemcpyAsync(stage, x_packed, sizeof(double) * packed, kin, h->stream));
@@ -493,15 +497,22 @@ int batch_solve(gis_context* h, double* x_packed, const double* b_packed, bool d
     hipLaunchKernelGGL((k_bsetup<Sell>), g, dim3(kWG), 0, h->stream, m, N, b, x, r, bv);
     GIS_HIP(h, hipGetLastError());
     const int block = std::max(1, std::min(h->sched.block_iters, 32));
-    if (use_graph) GIS_TRY(batch_graph(h, block, m, N, r, pb0, pb1, x, q, bv));
+    bool rest = true;   // systems are left to the loop below
+    if (resident) {   // p in pb0, the exchanged q from pb1 on
+        for (int s = 0; s < S; ++s) B.st_host[s].done = 0;
+        GIS_TRY(resident_batch(h, m, r, pb0, pb1, x));
+        rest = false;
+        for (int s = 0; s < S; ++s) rest = rest || !B.st_host[s].done;
+    }
+    if (rest && use_graph) GIS_TRY(batch_graph(h, block, m, N, r, pb0, pb1, x, q, bv));
     hipEvent_t ev_main = nullptr, ev_cap = nullptr;
-    if (use_graph) {
+    if (rest && use_graph) {
         GIS_HIP(h, hipEventCreateWithFlags(&ev_main, hipEventDisableTiming));
         GIS_HIP(h, hipEventCreateWithFlags(&ev_cap, hipEventDisableTiming));
     }
     long long launched = 0;
     int rc = kOK;
-    for (;;) {
+    while (rest) {
         if (use_graph) {
             // order the graph after the work already on the handle stream, and back
             if (hipEventRecord(ev_main, h->stream) != hipSuccess ||

@@ -106,6 +106,12 @@ struct BatchInfo {
     void* graph_key = nullptr;
     bool graph_selld = false;            // the SpMV layout the captured graph uses
     bool graph_split = false;            // the direction form the captured graph uses
+    // resident launches (gis_resident.hip): the workgroups' places launch by launch
+    // (res_first[l] .. res_first[l + 1]; empty: not laid out yet), tiles per
+    // workgroup, slot sets
+    DevMem res_blocks;
+    std::vector<int> res_first;
+    int res_tiles = 1, res_slots = 0;
 };
 
 // GAMG hierarchy (preconditioned CG).  Level 0 is the handle's own matrix;
@@ -392,6 +398,9 @@ template <typename T>
 struct Mat;
 bool resident_cg_fits(const gis_context* h);
 bool resident_bicg_fits(const gis_context* h);
+bool resident_batch_fits(const gis_context* h);
+int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, double* qx,
+                   double* x);
 int resident_cg(gis_context* h, const Mat<double>& m, double* r, double* p, double* qx, double* x,
                 bool* ran);
 int resident_bicg(gis_context* h, const Mat<double>& m, const Mat<double>& mt, double* r,

@@ -27,6 +27,7 @@
 #include <climits>
 #include <cmath>
 #include <mutex>
+#include <vector>
 
 #include "gis_kernels.hpp"
 
@@ -52,6 +53,12 @@ struct ResWs {
 };
 
 enum : int { kResWait = 0, kResGo = 1, kResLate = 2, kResNoFit = 3 };
+
+// A workgroup's place: workgroup g of the G that share one system, whose rows end
+// at row_end; row0 is the workgroup's first.
+struct ResPlace {
+    int row0, row_end, g, G;
+};
 
 template <int CTRL>
 __device__ __forceinline__ double dpp(double v) {
@@ -109,8 +116,8 @@ __device__ __forceinline__ double wave_total(double v) {
 
 // All workgroups of the launch, or none: true once gridDim.x have arrived.  A
 // workgroup that cannot take part (fits = false) gives up for all.  The verdict
-// of a launch that does not go ahead is left in KState::flag.
-__device__ __forceinline__ bool arrive_all(const ResWs& ws, bool fits, KState* st, int* sh) {
+// of a launch that does not go ahead is left in *verdict.
+__device__ __forceinline__ bool arrive_all(const ResWs& ws, bool fits, int* verdict, int* sh) {
     if (threadIdx.x == 0) {
         auto settle = [&](int to) {
             int expect = kResWait;
@@ -129,7 +136,7 @@ __device__ __forceinline__ bool arrive_all(const ResWs& ws, bool fits, KState* s
             if (wall_clock64() - t0 > ws.patience) settle(kResLate);
             __builtin_amdgcn_s_sleep(1);
         }
-        if (s != kResGo) st->flag = s;
+        if (s != kResGo) *verdict = s;
         *sh = s;
     }
     __syncthreads();
@@ -144,7 +151,7 @@ __device__ __forceinline__ bool arrive_all(const ResWs& ws, bool fits, KState* s
 // publication).  ok = false when the bounded wait ran out.
 template <int RPT, int NV>
 __device__ __forceinline__ void allreduce(const double (*part)[64 * RPT], const ResWs& ws,
-                                          unsigned phase, int fault, double (&t)[NV], bool& ok) {
+                                          const ResPlace& at, unsigned phase, int fault, double (&t)[NV], bool& ok) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
@@ -157,16 +164,16 @@ __device__ __forceinline__ void allreduce(const double (*part)[64 * RPT], const 
             for (int i = 0; i + h < RPT; i += 2 * h) e[i] = e[i] + e[i + h];
         t[v] = wave_total(e[0]);
     }
-    const int G = (int)gridDim.x;
+    const int G = at.G;
     ok = true;
     if (G == 1) return;
     double* set = ws.slot + (size_t)(phase % kResSets) * kResSlots;
-    double* own = set + (size_t)lane * kCopyStride + blockIdx.x;   // lane < kResCopies
+    double* own = set + (size_t)lane * kCopyStride + at.g;   // lane < kResCopies
     if (lane < kResCopies) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) st_agent(own + v * kResMaxGrid, t[v]);
     }
-    const double* mine = set + (size_t)(blockIdx.x % kResCopies) * kCopyStride;
+    const double* mine = set + (size_t)(at.g % kResCopies) * kCopyStride;
     const int limit = fault > 0 ? fault : kSlotSpins;
     double x[NV][4];
     for (int spins = 0;; ++spins) {
@@ -196,7 +203,7 @@ __device__ __forceinline__ void allreduce(const double (*part)[64 * RPT], const 
     }
     if (lane < kResCopies) {
         double* old = ws.slot + (size_t)((phase + 2) % kResSets) * kResSlots +
-                      (size_t)lane * kCopyStride + blockIdx.x;
+                      (size_t)lane * kCopyStride + at.g;
         slot_clear(old);
         slot_clear(old + kResMaxGrid);
     }
@@ -242,8 +249,8 @@ struct ResRows {
 // slot columns.  val / valT: the slot values of A, and of A^T (M = 2) from mt.
 // Ends with a workgroup barrier, the LDS vectors free.
 template <int RPT, int M, bool TAB, bool ALONE>
-__device__ __forceinline__ void res_rows(const Mat<double>& m, const Mat<double>& mt, int N,
-                                         unsigned char* lds, int* n_halo, int* wsum,
+__device__ __forceinline__ void res_rows(const Mat<double>& m, const Mat<double>& mt,
+                                         const ResPlace& place, unsigned char* lds, int* n_halo, int* wsum,
                                          ResRows<RPT, M, ALONE>& rows,
                                          double (&val)[RPT][kResEntries],
                                          double (&valT)[M == 2 ? RPT : 1][kResEntries]) {
@@ -251,7 +258,7 @@ __device__ __forceinline__ void res_rows(const Mat<double>& m, const Mat<double>
     constexpr int K = kResEntries;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row0 = (int)blockIdx.x * G::kRows;
+    const int row0 = place.row0, N = place.row_end;
     const int nloc = min(G::kRows, N - row0);
     const int nslices = (N + kSlice - 1) / kSlice;
     int* hash = reinterpret_cast<int*>(lds);
@@ -410,7 +417,8 @@ __device__ __forceinline__ bool poll_halo(const ResRows<RPT, M, ALONE>& rows, co
 // The workgroup's slots and exchanged rows emptied, then the handshake.
 template <int RPT, int M, bool ALONE>
 __device__ __forceinline__ bool res_start(const ResRows<RPT, M, ALONE>& rows, const ResWs& ws,
-                                          double* qx, size_t n, int row, KState* st, int* sh) {
+                                          const ResPlace& at, double* qx, size_t n, int row,
+                                          int* verdict, int* sh) {
     using G = ResGeom<RPT, M, ALONE>;
     if constexpr (ALONE) {
         __syncthreads();
@@ -424,18 +432,18 @@ __device__ __forceinline__ bool res_start(const ResRows<RPT, M, ALONE>& rows, co
     const int tid = threadIdx.x;
     if (tid < kResSets * kResCopies) {
         double* s = ws.slot + (size_t)(tid / kResCopies) * kResSlots +
-                    (size_t)(tid % kResCopies) * kCopyStride + blockIdx.x;
+                    (size_t)(tid % kResCopies) * kCopyStride + at.g;
         slot_clear(s);
         slot_clear(s + kResMaxGrid);
     }
     order_release();
     __syncthreads();
-    return arrive_all(ws, rows.nh <= G::kHalo, st, sh);
+    return arrive_all(ws, rows.nh <= G::kHalo, verdict, sh);
 }
 
-__device__ __forceinline__ void res_hist(const KState* st, double* hist, int hist_cap, int detail,
-                                         int k, double norm) {
-    if (blockIdx.x == 0 && k < hist_cap)
+__device__ __forceinline__ void res_hist(const KState* st, const ResPlace& at, double* hist,
+                                         int hist_cap, int detail, int k, double norm) {
+    if (at.g == 0 && k < hist_cap)
         hist[k] = detail ? (double)(wall_clock64() - st->t0) * st->tick : norm;
 }
 
@@ -448,24 +456,24 @@ __device__ __forceinline__ void res_hist(const KState* st, double* hist, int his
 // buffers rotate: whoever has completed the first reduction of iteration k knows
 // that every workgroup is done with q of k - 1, and empties its rows there; they
 // are written again in iteration k + 2.
+//
+// n: the vectors' length (q buffers lie n apart).  verdict: arrive_all's.
 template <int RPT, bool TAB, bool ALONE>
-__global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double* __restrict__ r,
-                                                   double* __restrict__ p, double* __restrict__ qx,
-                                                   double* __restrict__ x, KState* st, ResWs ws,
-                                                   int chunk) {
+__device__ __forceinline__ void cg_res(const Mat<double>& m, const ResPlace& at, size_t n,
+                                       double* __restrict__ r, double* __restrict__ p,
+                                       double* __restrict__ qx, double* __restrict__ x,
+                                       KState* st, const ResWs& ws, int chunk, int* verdict) {
     using G = ResGeom<RPT, 1, ALONE>;
     constexpr int H = G::kHpt;
     __shared__ __attribute__((aligned(16))) unsigned char lds[G::kBytes];
     __shared__ double part[1][64 * RPT];
     __shared__ double bc[2];
     __shared__ int bci, n_halo, wsum[kResWG / 64];
-    if (st->done) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row0 = (int)blockIdx.x * G::kRows;
+    const int row0 = at.row0, N = at.row_end;
     const int nloc = min(G::kRows, N - row0);
     const int li0 = w * RPT * kSlice + lane;   // the thread's rows: li0, li0 + 64, ...
-    const size_t n = (size_t)N;
     const int k0 = st->k, fault = st->slot_fault;
     const double error = st->error;
     const long long max_steps = st->max_steps, min_steps = st->min_steps;
@@ -476,7 +484,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
 
     ResRows<RPT, 1, ALONE> rows;
     double val[RPT][kResEntries], none[1][kResEntries];
-    res_rows<RPT, 1, TAB, ALONE>(m, m, N, lds, &n_halo, wsum, rows, val, none);
+    res_rows<RPT, 1, TAB, ALONE>(m, m, at, lds, &n_halo, wsum, rows, val, none);
     double* sp = reinterpret_cast<double*>(lds);
     if (tid == 0) sp[G::kZero] = 0.0;
     double rv[RPT], xv[RPT], rh[H > 0 ? H : 1];
@@ -495,7 +503,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
             sp[G::kRows + j * kResWG + tid] =
                 rows.hcol[j] >= 0 && k0 > 0 ? p[rows.hcol[j]] : 0.0;
     }
-    if (!res_start(rows, ws, qx, n, row0 + li0, st, &bci)) return;
+    if (!res_start(rows, ws, at, qx, n, row0 + li0, verdict, &bci)) return;
 
     unsigned phase = 0;
     bool stop = false, ok = true;
@@ -531,7 +539,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
         __syncthreads();
         if (w == 0) {
             double t[1];
-            allreduce<RPT, 1>(part, ws, phase, fault, t, ok);
+            allreduce<RPT, 1>(part, ws, at, phase, fault, t, ok);
             alpha = rho / t[0];
             if (lane == 0) {
                 bc[0] = alpha;
@@ -555,7 +563,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
         __syncthreads();
         if (w == 0) {
             double t[1];
-            allreduce<RPT, 1>(part, ws, phase, fault, t, ok);
+            allreduce<RPT, 1>(part, ws, at, phase, fault, t, ok);
             rho1 = rho;
             rho = t[0];
             beta = rho / rho1;
@@ -564,7 +572,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
                 bc[1] = beta;
                 bci = !ok ? 2
                           : ((!(norm > error) || k >= max_steps) && k >= min_steps) ? 1 : 0;
-                if (ok) res_hist(st, hist, hist_cap, detail, k, norm);
+                if (ok) res_hist(st, at, hist, hist_cap, detail, k, norm);
             }
         }
         ++phase;
@@ -604,7 +612,7 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
             p[row0 + li] = sp[li];
         }
     }
-    if (blockIdx.x == 0 && tid == 0) {
+    if (at.g == 0 && tid == 0) {
         st->k = k;
         st->norm = norm;
         st->rho0 = rho;
@@ -613,6 +621,43 @@ __global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double*
         st->beta = beta;
         if (stop) st->done = 1;
     }
+}
+
+template <int RPT, bool TAB, bool ALONE>
+__global__ __launch_bounds__(kResWG) void k_cg_res(Mat<double> m, int N, double* __restrict__ r,
+                                                   double* __restrict__ p, double* __restrict__ qx,
+                                                   double* __restrict__ x, KState* st, ResWs ws,
+                                                   int chunk) {
+    if (st->done) return;
+    const ResPlace at{(int)blockIdx.x * kResWG * RPT, N, (int)blockIdx.x, (int)gridDim.x};
+    cg_res<RPT, TAB, ALONE>(m, at, (size_t)N, r, p, qx, x, st, ws, chunk, &st->flag);
+}
+
+// Several systems of a batch in one launch: block b's place, system and slots.
+struct ResBlock {
+    ResPlace at;
+    int sys, slot;
+};
+
+template <int RPT>
+__global__ __launch_bounds__(kResWG) void k_bcg_res(Mat<double> m, size_t n,
+                                                    double* __restrict__ r,
+                                                    double* __restrict__ p,
+                                                    double* __restrict__ qx,
+                                                    double* __restrict__ x, KState* states,
+                                                    const ResBlock* __restrict__ blocks, ResWs ws,
+                                                    int chunk) {
+    const ResBlock b = blocks[blockIdx.x];
+    KState* st = states + b.sys;
+    if (st->done) {   // the others wait for this workgroup too
+        __shared__ int verdict;
+        (void)arrive_all(ws, true, &ws.sync[2], &verdict);
+        return;
+    }
+    ws.slot += (size_t)b.slot * kResSets * kResSlots;
+    cg_res<RPT, false, false>(m, b.at, n, r, p, qx, x, st, ws, chunk, &ws.sync[2]);
+    // x is complete: nothing is left to k_bcg_flush
+    if (b.at.g == 0 && threadIdx.x == 0 && st->k > 0) st->flag = 1;
 }
 
 // BiCG (k_bicg1, k_bicg2<P, 0>) in the same way, with A's slots from m and A^T's
@@ -636,7 +681,8 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
     if (st->done) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row0 = (int)blockIdx.x * G::kRows;
+    const ResPlace at{(int)blockIdx.x * G::kRows, N, (int)blockIdx.x, (int)gridDim.x};
+    const int row0 = at.row0;
     const int nloc = min(G::kRows, N - row0);
     const bool in = tid < nloc;
     const int row = row0 + tid;
@@ -651,7 +697,7 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
 
     ResRows<1, 2, ALONE> rows;
     double val[1][kResEntries], valT[1][kResEntries];
-    res_rows<1, 2, TAB, ALONE>(m, mt, N, lds, &n_halo, wsum, rows, val, valT);
+    res_rows<1, 2, TAB, ALONE>(m, mt, at, lds, &n_halo, wsum, rows, val, valT);
     double* sp = reinterpret_cast<double*>(lds);
     double* sps = sp + G::kZero + 1;
     if (tid == 0) sp[G::kZero] = sps[G::kZero] = 0.0;
@@ -670,7 +716,7 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
             sps[h] = c >= 0 && k0 > 0 ? ps[c] : 0.0;
         }
     }
-    if (!res_start(rows, ws, qx, n, row, st, &bci)) return;
+    if (!res_start(rows, ws, at, qx, n, row, &st->flag, &bci)) return;
 
     unsigned phase = 0;
     bool stop = false, ok = true, broke = false;
@@ -704,7 +750,7 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
         __syncthreads();
         if (w == 0) {
             double t[1];
-            allreduce<1, 1>(part, ws, phase, fault, t, ok);
+            allreduce<1, 1>(part, ws, at, phase, fault, t, ok);
             xi = rho / t[0];
             if (lane == 0) {
                 bc[0] = xi;
@@ -734,7 +780,7 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
         __syncthreads();
         if (w == 0) {
             double t[2];
-            allreduce<1, 2>(part, ws, phase, fault, t, ok);
+            allreduce<1, 2>(part, ws, at, phase, fault, t, ok);
             norm = sqrt(t[0]);
             const bool end = (norm < error || k >= max_steps) && k >= min_steps;
             if (!end) {
@@ -745,7 +791,7 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
             if (lane == 0) {
                 bc[1] = beta;
                 bci = !ok ? 2 : end ? 1 : 0;
-                if (ok) res_hist(st, hist, hist_cap, detail, k, norm);
+                if (ok) res_hist(st, at, hist, hist_cap, detail, k, norm);
             }
         }
         ++phase;
@@ -835,6 +881,10 @@ int run_resident(gis_context* h, Launch&& launch, bool* ran) {
     }
 }
 
+__global__ void k_res_reset_all(int* sync, int n) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) sync[i] = 0;
+}
+
 // TAB form of the pattern; false: it takes no resident form.  The int32 slots
 // serve where some slice has no offset table, or a long one.
 bool res_form(const gis_context* h, bool* tab) {
@@ -902,6 +952,101 @@ int resident_bicg(gis_context* h, const Mat<double>& m, const Mat<double>& mt, d
         if (g.x == 1) tab ? go(k_bicg_res<true, true>) : go(k_bicg_res<false, true>);
         else tab ? go(k_bicg_res<true, false>) : go(k_bicg_res<false, false>);
     }, ran);
+}
+
+// Measured against one launch per stage for the whole batch (edges, tiles in all):
+// 64 systems of 8-24, 364: 4.67 -> 1.43 ms; 8 of 16-64, 422: 9.9 -> 4.3; 64 of 20-40,
+// 1980: 18.3 -> 9.2; 32 of 16-64, 2994: 35.3 -> 31.0; 64 of 16-64, 5735: 60.2 -> 57.7;
+// 20 of 50-64, 3657: 44.0 -> 44.7, where both run at the chip's rate.
+// A batch's systems as resident launches, each of as many systems as fit the chip
+// together (largest first, so that those of one launch take about as long).
+// Systems that are not done afterwards have not been started: the caller's loop
+// takes them.
+int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, double* qx,
+                   double* x) {
+    BatchInfo& B = h->batch;
+    if (!resident_batch_fits(h)) return kOK;
+    const int n_cu = std::min(h->n_cu, kResMaxGrid), S = B.S;
+    if (B.res_first.empty()) {   // once per pattern
+        std::vector<int> sys(S);
+        long long tiles = 0;
+        for (int i = 0; i < S; ++i) {
+            sys[i] = i;
+            tiles += B.tile0[i + 1] - B.tile0[i];
+        }
+        B.res_tiles = tiles <= n_cu ? 1 : 2;
+        const auto groups = [&](int i) {
+            return (B.tile0[i + 1] - B.tile0[i] + B.res_tiles - 1) / B.res_tiles;
+        };
+        std::stable_sort(sys.begin(), sys.end(),
+                         [&](int a, int b) { return groups(a) > groups(b); });
+        std::vector<ResBlock> blocks;
+        std::vector<int> first;
+        int slot = 0, slots = 0;
+        for (int i : sys) {
+            const int G = groups(i);
+            if (first.empty() || (int)blocks.size() - first.back() + G > n_cu) {
+                first.push_back((int)blocks.size());
+                slot = 0;
+            }
+            for (int g = 0; g < G; ++g)
+                blocks.push_back(ResBlock{{B.pad_off[i] + g * B.res_tiles * kTile,
+                                           B.pad_off[i] + B.n[i], g, G}, i, slot});
+            slots = std::max(slots, ++slot);
+        }
+        first.push_back((int)blocks.size());
+        GIS_HIP(h, B.res_blocks.ensure(sizeof(ResBlock) * blocks.size()));
+        GIS_HIP(h, hipMemcpyAsync(B.res_blocks.p, blocks.data(), sizeof(ResBlock) * blocks.size(),
+                                  hipMemcpyHostToDevice, h->stream));
+        GIS_HIP(h, hipStreamSynchronize(h->stream));   // blocks is a host temporary
+        B.res_slots = slots;
+        B.res_first = first;
+    }
+    std::unique_lock<std::mutex> lock(g_resident[h->device], std::try_to_lock);
+    if (!lock.owns_lock()) return kOK;
+    const int L = (int)B.res_first.size() - 1;
+    const size_t n_slot = (size_t)B.res_slots * kResSets * kResSlots;
+    GIS_HIP(h, h->res_mem.ensure(sizeof(double) * n_slot + sizeof(int) * 4 * (size_t)L));
+    double* slot = h->res_mem.as<double>();
+    int* sync = reinterpret_cast<int*>(slot + n_slot);
+    const double tick = h->wall_tick > 0.0 ? h->wall_tick : 1e-8;
+    std::vector<int> verdict(4 * (size_t)L);
+    for (int late = 0; late <= 1000; ++late) {
+        hipLaunchKernelGGL(k_res_reset_all, dim3(1), dim3(kWG), 0, h->stream, sync, 4 * L);
+        for (int l = 0; l < L; ++l) {
+            const ResWs ws{slot, sync + 4 * l, (long long)(5e-3 / tick)};
+            const dim3 g((unsigned)(B.res_first[l + 1] - B.res_first[l]));
+            const auto go = [&](auto k) {
+                hipLaunchKernelGGL(k, g, dim3(kResWG), 0, h->stream, m, (size_t)h->N, r, p, qx, x,
+                                   B.st.as<KState>(), B.res_blocks.as<ResBlock>() + B.res_first[l],
+                                   ws, kResChunk);
+            };
+            B.res_tiles == 1 ? go(k_bcg_res<1>) : go(k_bcg_res<2>);
+        }
+        GIS_HIP(h, hipGetLastError());
+        GIS_HIP(h, hipMemcpyAsync(B.st_host, B.st.p, sizeof(KState) * S, hipMemcpyDeviceToHost,
+                                  h->stream));
+        GIS_HIP(h, hipMemcpyAsync(verdict.data(), sync, sizeof(int) * 4 * (size_t)L,
+                                  hipMemcpyDeviceToHost, h->stream));
+        GIS_HIP(h, hipStreamSynchronize(h->stream));
+        for (int l = 0; l < L; ++l)
+            if (verdict[4 * l + 2] == kResNoFit) h->res_unfit = true;
+        // a system that a chunk left unfinished goes on in its resident form
+        bool open = false;
+        for (int i = 0; i < S; ++i) open = open || (!B.st_host[i].done && B.st_host[i].k > 0);
+        if (!open) return kOK;
+    }
+    return fail(h, kErrSync, "the batch's grid could not be made resident again");
+}
+
+bool resident_batch_fits(const gis_context* h) {
+    bool tab;
+    if (!res_form(h, &tab) || h->lay_max_row > kResEntries) return false;
+    const BatchInfo& B = h->batch;
+    const int n_cu = std::min(h->n_cu, kResMaxGrid);
+    int most = 0;
+    for (int i = 0; i < B.S; ++i) most = std::max(most, B.tile0[i + 1] - B.tile0[i]);
+    return most <= 2 * n_cu;
 }
 
 }  // namespace gis

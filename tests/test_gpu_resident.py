@@ -146,3 +146,53 @@ def test_infinite_and_nan_inputs(gpu):
             assert st == st1
             np.testing.assert_array_equal(hist, hist1)
             np.testing.assert_array_equal(x, x1)
+
+
+@pytest.mark.parametrize("edges", [[1, 2, 10, 11, 13], [40, 64, 3, 65, 17, 30, 30, 30],
+                                   [20] * 40 + [8] * 30])
+def test_batch(gpu, edges):
+    """One launch, several launches with systems of one and of two tiles per
+    workgroup, and many small systems: every system its own solve's bits."""
+    systems = [mesh.laplacian(n, seed=50 + i, shift=1e-3) for i, n in enumerate(edges)]
+    err = np.array([1e-6 * np.linalg.norm(s.b) for s in systems])
+    b = np.concatenate([s.b for s in systems])
+
+    def run(g):
+        return g.batch_solve(b, None, err, 70)
+    gpu.batch_set_systems(systems)
+    for _ in range(2):
+        x, it, nf, st = run(gpu)
+    gpu.batch_set_systems(systems)
+    x1, it1, nf1, st1 = stages(gpu, run)
+    np.testing.assert_array_equal(it, it1)
+    np.testing.assert_array_equal(nf, nf1)
+    np.testing.assert_array_equal(x, x1)
+    off = 0
+    for i, s in enumerate(systems):
+        if s.n_cells <= 2200:
+            ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, err[i], 70)
+            assert it[i] == ref.iterations and nf[i] == ref.hist[-1]
+            np.testing.assert_array_equal(x[off:off + s.n_cells], ref.x)
+        off += s.n_cells
+
+
+def test_batch_mixed_fit(gpu):
+    """More iterations than a chunk, and a batch one of whose systems has long rows
+    (the whole batch then runs stage by stage)."""
+    small = [mesh.laplacian(n, seed=n, shift=1e-3) for n in (20, 3, 9)]
+    b = np.concatenate([s.b for s in small])
+    gpu.batch_set_systems(small)
+    x, it, nf, st = gpu.batch_solve(b, None, -1.0, 2100)
+    ref = O.solve("CG", O.ldu2csr(small[0]), small[0].b, small[0].x0, -1.0, 2100)
+    assert it[0] == ref.iterations == 2100 and nf[0] == ref.hist[-1]
+    np.testing.assert_array_equal(x[:8000], ref.x)
+    mixed = small + [mesh.random_ldu(900, 9000, seed=1, symmetric=True)]
+    b = np.concatenate([s.b for s in mixed])
+    gpu.batch_set_systems(mixed)
+    x, it, nf, st = gpu.batch_solve(b, None, 1e-8, 300)
+    off = 0
+    for i, s in enumerate(mixed):
+        ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, 1e-8, 300)
+        assert it[i] == ref.iterations
+        np.testing.assert_array_equal(x[off:off + s.n_cells], ref.x)
+        off += s.n_cells
