@@ -399,106 +399,124 @@ struct TailLevel {
     T* t;
 };
 
-constexpr int kTail = 256;        // one workgroup runs a level in ~10 us per step: only tiny levels
+// Cells of the tail's first level.  One workgroup waits for each step's matrix
+// entries alone, so larger levels stay launches of their own (GAMG iteration at
+// 64^3, 45^3 in FP32, 128^3 with 256 / 512 / 1024: 164, 176, 347 / 173, 162, 348 / 180,
+// 161, 350 us).
+constexpr int kTail = 256;
+constexpr int kTailCells = 1024;  // of all its levels together
 constexpr int kTailThreads = 1024;
+constexpr int kTailBatch = 16;
 
-// Row i of a tail level: a batch's column and value loads, then its gathers,
+// Row i of a tail level times the LDS vector x: a batch's column and value loads
 // are in flight together; the products are summed one by one in storage order.
 template <typename T>
 __device__ __forceinline__ T csr_row(const TailLevel<T>& L, int i, const T* x) {
     const int a = L.rowptr[i], b = L.rowptr[i + 1];
     T s = T(0);
-    for (int j = a; j < b; j += 8) {
-        int c[8];
-        T v[8], xv[8];
+    for (int j = a; j < b; j += kTailBatch) {
+        int c[kTailBatch];
+        T v[kTailBatch];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < kTailBatch; ++u) {
             const int q = min(j + u, b - 1);
             c[u] = L.col[q];
             v[u] = L.val[q];
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) xv[u] = x[c[u]];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (j + u < b) s = s + v[u] * xv[u];
+        for (int u = 0; u < kTailBatch; ++u) {
+            const T t = s + v[u] * x[c[u]];
+            s = j + u < b ? t : s;
+        }
     }
     return s;
 }
 
 // On entry lv[0].r holds the rhs and lv[0].z its first sweep from zero; on
-// exit lv[0].z holds the cycle's result.
+// exit lv[0].z holds the cycle's result.  Every level's vectors, and the dense
+// inverse (transposed, so that a wave reads it without bank conflicts), stay in
+// LDS: a step waits for its matrix entries only (64^3 180 -> 164 us per GAMG
+// iteration against vectors in global memory and 64 dependent loads a dense row).
 template <typename T>
 __global__ __launch_bounds__(kTailThreads) void k_vc_tail(const TailLevel<T>* __restrict__ lv,
                                                           int nl, int nu, T cscale,
                                                           const T* __restrict__ ainv,
                                                           int dense_n, const KState* st) {
     if (st->done) return;
+    __shared__ T vr[kTailCells], vz[2][kTailCells], vt[kTailCells];
+    __shared__ T inv[kDense * kDense];
     const int tid = threadIdx.x;
     const int nt = blockDim.x;
-    T* cur[kAmgLevels];
+    for (int e = tid; e < dense_n * dense_n; e += nt)
+        inv[e % dense_n * dense_n + e / dense_n] = ainv[e];
+    for (int i = tid; i < lv[0].n; i += nt) {
+        vr[i] = lv[0].r[i];
+        vz[0][i] = lv[0].z[i];
+    }
+    __syncthreads();
+    unsigned which = 0;   // bit l: level l's z is in vz[1]
+    int off = 0;          // of the level in the LDS vectors
     for (int l = 0; l + 1 < nl; ++l) {
         const TailLevel<T>& L = lv[l];
-        T* z = L.z;
-        T* z2 = L.z2;
+        int w = 0;
         for (int s = 1; s < nu; ++s) {
             for (int i = tid; i < L.n; i += nt)
-                z2[i] = fmaT(L.sm[i], L.r[i] - csr_row(L, i, z), z[i]);
+                vz[w ^ 1][off + i] = fmaT(L.sm[i], vr[off + i] - csr_row(L, i, vz[w] + off),
+                                          vz[w][off + i]);
             __syncthreads();
-            T* tmp = z;
-            z = z2;
-            z2 = tmp;
+            w ^= 1;
         }
-        for (int i = tid; i < L.n; i += nt) L.t[i] = L.r[i] - csr_row(L, i, z);
+        for (int i = tid; i < L.n; i += nt)
+            vt[off + i] = vr[off + i] - csr_row(L, i, vz[w] + off);
         __syncthreads();
         const TailLevel<T>& C = lv[l + 1];
+        const int next = off + L.n;
         for (int c = tid; c < C.n; c += nt) {
             const int p0 = L.mptr[c], p1 = L.mptr[c + 1];
             T s = T(0);
             for (int p = p0; p < p1; p += 4) {
-                T v[4];
+                int m[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = L.t[L.mlist[min(p + u, p1 - 1)]];
+                for (int u = 0; u < 4; ++u) m[u] = L.mlist[min(p + u, p1 - 1)];
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    if (p + u < p1) s = s + v[u];
+                    if (p + u < p1) s = s + vt[off + m[u]];
             }
-            C.r[c] = s;
-            C.z[c] = C.sm[c] * s;
+            vr[next + c] = s;
+            vz[0][next + c] = C.sm[c] * s;
         }
         __syncthreads();
-        cur[l] = z;
+        which |= (unsigned)w << l;
+        off = next;
     }
     const TailLevel<T>& E = lv[nl - 1];
     if (dense_n) {
         for (int i = tid; i < E.n; i += nt) {
             T s = T(0);
-            for (int j = 0; j < E.n; ++j) s = s + ainv[i * E.n + j] * E.r[j];
-            E.z[i] = s;
+            for (int j = 0; j < E.n; ++j) s = s + inv[j * dense_n + i] * vr[off + j];
+            vz[0][off + i] = s;
         }
         __syncthreads();
     }
-    const T* zc = E.z;
+    int wc = 0, coff = off;   // where the coarser level's z is
     for (int l = nl - 2; l >= 0; --l) {
         const TailLevel<T>& L = lv[l];
-        T* z = cur[l];
-        T* z2 = (z == L.z) ? L.z2 : L.z;
-        for (int i = tid; i < L.n; i += nt) z[i] = fmaT(cscale, zc[L.agg[i]], z[i]);
+        off = coff - L.n;
+        int w = (which >> l) & 1u;
+        for (int i = tid; i < L.n; i += nt)
+            vz[w][off + i] = fmaT(cscale, vz[wc][coff + L.agg[i]], vz[w][off + i]);
         __syncthreads();
         for (int s = 0; s < nu; ++s) {
             for (int i = tid; i < L.n; i += nt)
-                z2[i] = fmaT(L.sm[i], L.r[i] - csr_row(L, i, z), z[i]);
+                vz[w ^ 1][off + i] = fmaT(L.sm[i], vr[off + i] - csr_row(L, i, vz[w] + off),
+                                          vz[w][off + i]);
             __syncthreads();
-            T* tmp = z;
-            z = z2;
-            z2 = tmp;
+            w ^= 1;
         }
-        if (z != L.z) {
-            for (int i = tid; i < L.n; i += nt) L.z[i] = z[i];
-            __syncthreads();
-        }
-        zc = L.z;
+        wc = w;
+        coff = off;
     }
+    for (int i = tid; i < lv[0].n; i += nt) lv[0].z[i] = vz[wc][i];
 }
 
 // z = Ainv r on the last level (n <= kDense)
@@ -826,11 +844,12 @@ int amg_values(gis_context* h) {
     // the coarse tail (levels of at most kTail cells below the finest) as one workgroup
     A.tail_start = 0;
     A.tail_levels = 0;
-    for (size_t l = 1; l < A.lv.size(); ++l)
-        if (A.lv[l].n <= kTail) {
-            A.tail_start = (int)l;
-            break;
-        }
+    long long cells = 0;
+    for (size_t l = A.lv.size() - 1; l >= 1; --l) {
+        cells += A.lv[l].n;
+        if (A.lv[l].n > kTail || cells > kTailCells) break;
+        A.tail_start = (int)l;
+    }
     if (A.tail_start) {
         std::vector<TailLevel<double>> meta;
         for (size_t l = A.tail_start; l < A.lv.size(); ++l) {
