@@ -209,6 +209,7 @@ struct gis_context {
     // (sym_layout), used while the values are bitwise symmetric (sym_values) and
     // the caller has not switched it off (sym_enable)
     gis::DevMem syma, symb, dsv;
+    gis::DevMem sym_flag;       // the symmetry check's verdict
     gis::DevMem symx;   // per table entry {offset, syma, symb, 0}: one 16-byte load a slot
     long long n_sym_slots = 0;
     bool sym_layout = false;

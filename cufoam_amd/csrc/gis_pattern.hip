@@ -789,7 +789,8 @@ int gather_values(gis_context* h) {
     h->sym_values = false;
     if (h->sym_layout) {
         GIS_TRY(sym_compact<double>(h, h->dval, h->dsv));
-        DevMem flag;
+        // kept: allocating and freeing it took 16 us of every set_values (16^3: 105 -> 89)
+        DevMem& flag = h->sym_flag;
         GIS_HIP(h, flag.ensure(sizeof(int)));
         GIS_HIP(h, hipMemsetAsync(flag.p, 0, sizeof(int), h->stream));
         const int S = (int)h->lay_slices;
