@@ -202,6 +202,7 @@ struct gis_context {
     long long lay_slices = 0, lay_table_slices = 0, lay_table_entries = 0;
     long long lay_byte_mask_slices = 0, lay_untabled_slots = 0;
     int lay_max_table = 0, lay_max_row = 0;     // longest offset table, longest row
+    int lay_max_offset = 0;                     // farthest offset of the tables
     gis::DevMem dval, dvalT, dval32, dval32T;
     // symmetric storage of the SellD layout (every slice tabled): the FP64 slot
     // values of the table entries with column offset >= 0 only (dsv), and per

@@ -31,6 +31,7 @@ struct Mat {
     // per table entry {offset, value bases}, and the kept slot values; null: full slots
     const int4* symx;
     const T* dsv;
+    int chunk = 0;   // tiles an XCD takes at a time (chunk_tile); 0: one
 };
 
 // ---------------------------------------------------------------------------
@@ -159,6 +160,20 @@ __device__ __forceinline__ int xcd_tile(int i, int G) {
     return x * q + min(x, r) + j;
 }
 
+// Workgroup i's tile when each XCD takes c consecutive tiles at a time (c <= 0: one,
+// the dispatch order).  Tiles 8 c apart then share an XCD, whose L2 holds what a
+// row's far neighbours need: c is an eighth of the farthest offset's distance in
+// tiles where that is no multiple of 8 (mat_chunk).  Past the last whole span of 8 c
+// tiles the dispatch order goes on.  A group's last tile may go out up to 8 c
+// workgroups early; its collector waits for those few.
+__device__ __forceinline__ int chunk_tile(int i, int T, int c) {
+    if (c <= 0) return i;
+    const int span = kXcds * c;
+    if (i >= T / span * span) return i;
+    const int x = i % kXcds, j = i / kXcds;
+    return (j / c * kXcds + x) * c + j % c;
+}
+
 // Row range of a workgroup tile.  TileRows(N): tile = workgroup index (best for
 // the SpMV-carrying kernels and the updates that follow them, measured);
 // StreamRows(N): XCD-contiguous tiles.
@@ -185,6 +200,10 @@ struct SuperTile {
     __device__ SuperTile(int N, bool stream) {
         const int s = stream ? xcd_tile((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
         tile0 = s * C;
+        nt = min(C, tiles_of(N) - tile0);
+    }
+    __device__ SuperTile(int N, int chunk) {
+        tile0 = chunk_tile((int)blockIdx.x, (int)gridDim.x, chunk) * C;
         nt = min(C, tiles_of(N) - tile0);
     }
 };
@@ -263,7 +282,7 @@ __global__ __launch_bounds__(kWG) void k_cg1s(Mat<double> m, int N,
     __shared__ typename P::template Shared<double> sh;
     __shared__ double sh_y[kTile];
     __shared__ RedShared shr;
-    const SuperTile<C> sup(N, false);
+    const SuperTile<C> sup(N, m.chunk);
     const double* p = ((st->k + 1) & 1) ? pb1 : pb0;
     double leaf[C][1];
 #pragma unroll
@@ -342,6 +361,19 @@ inline dim3 super_grid(int N, int C) { return dim3((unsigned)((tiles_of(N) + C -
         } break;                          \
     }
 
+// Tiles an XCD takes at a time in k_cg1s and k_mx1 (chunk_tile), from the farthest
+// table offset of P tiles: P / 8, rounded, from 3 up and where P is not a multiple
+// of 8 already.  Per iteration, without / with (FP64 CG and mixed): 160^3 99.4 /
+// 91.3 and 57.8 / 56.0 us, 200^3 189.3 / 184.9 and 103.1 / 97.6, 245^3 351.1 / 348.4
+// and 184.3 / 172.3; not below (140^3, P 19: 71.8 / 71.7 and 44.3 / 44.7) nor at
+// 256^3 (P 64: 376.5 / 377.3 and 192.9 / 194.2).
+inline int mat_chunk(const gis_context* h) {
+    constexpr int kSpan = kXcds * kTile;
+    const int off = h->lay_max_offset;
+    const int c = (off + kSpan / 2) / kSpan;
+    return c >= 3 && off % kSpan != 0 ? c : 0;
+}
+
 inline Mat<double> mat64(const gis_context* h) {
     const bool sym = use_sym(h);
     return Mat<double>{h->rowptr.as<int>(), h->col.as<int>(), h->val.as<double>(),
@@ -350,7 +382,8 @@ inline Mat<double> mat64(const gis_context* h) {
                        h->sflag.as<unsigned char>(),
                        h->ooff.as<int>(), h->doffs.as<int>(), h->dmask.as<unsigned>(),
                        h->dval.as<double>(), h->dmask8.as<unsigned char>(),
-                       sym ? h->symx.as<int4>() : nullptr, sym ? h->dsv.as<double>() : nullptr};
+                       sym ? h->symx.as<int4>() : nullptr, sym ? h->dsv.as<double>() : nullptr,
+                       mat_chunk(h)};
 }
 
 inline Mat<double> mat64T(const gis_context* h) {
@@ -379,7 +412,8 @@ inline Mat<float> mat32(const gis_context* h) {
                       h->sres.as<signed char>(), h->sbase.as<int>(),
                       h->sflag.as<unsigned char>(),
                       h->ooff.as<int>(), h->doffs.as<int>(), h->dmask.as<unsigned>(),
-                      h->dval32.as<float>(), h->dmask8.as<unsigned char>(), nullptr, nullptr};
+                      h->dval32.as<float>(), h->dmask8.as<unsigned char>(), nullptr, nullptr,
+                      mat_chunk(h)};
 }
 
 // Iterations the host may launch: the cap, or min_steps when that is larger

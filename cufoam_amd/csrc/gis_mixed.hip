@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kWG) void k_mx1(Mat<float> m, int N, const float* _
     __shared__ typename P::template Shared<float> sh;
     __shared__ float sh_y[kTile];
     __shared__ RedShared shr;
-    const SuperTile<C> sup(N, false);
+    const SuperTile<C> sup(N, m.chunk);
     const int k = st->k + 1;
     const int flag = st->flag;
     const bool first = (flag & F_RESTART) != 0;

@@ -225,21 +225,27 @@ __global__ __launch_bounds__(kBlk) void k_selld_union(int N, int S,
     }
 }
 
-// longest[0]: the longest offset table, longest[1]: the longest row of the pattern
+// longest[0]: the longest offset table, [1]: the longest row of the pattern, [2]: the
+// farthest (positive) offset of the tables
 __global__ __launch_bounds__(kBlk) void k_longest(int S, const int* __restrict__ ucount,
-                                                  const int* __restrict__ soff, int* longest) {
-    int u = 0, len = 0;
+                                                  const int* __restrict__ soff,
+                                                  const int* __restrict__ tmp_offs,
+                                                  int* longest) {
+    int u = 0, len = 0, far = 0;
     for (int s = blockIdx.x * kBlk + threadIdx.x; s < S; s += gridDim.x * kBlk) {
         u = max(u, ucount[s]);
         len = max(len, (soff[s + 1] - soff[s]) / kSlice);
+        if (ucount[s] > 0) far = max(far, tmp_offs[(size_t)s * 32 + ucount[s] - 1]);
     }
     for (int o = 32; o > 0; o >>= 1) {
         u = max(u, __shfl_xor(u, o, 64));
         len = max(len, __shfl_xor(len, o, 64));
+        far = max(far, __shfl_xor(far, o, 64));
     }
     if ((threadIdx.x & 63) == 0) {
         atomicMax(&longest[0], u);
         atomicMax(&longest[1], len);
+        atomicMax(&longest[2], far);
     }
 }
 
@@ -660,14 +666,14 @@ int build_pattern(gis_context* h, int N, int M, const int* d_la, const int* d_ua
     // column-offset tables (SellD)
     {
         DevMem ucount, tmp_offs;
-        // ucount[0..S]: table sizes (ucount[S] = 0 for the scan); ucount[S+1..S+5]:
+        // ucount[0..S]: table sizes (ucount[S] = 0 for the scan); ucount[S+1..S+6]:
         // the layout counts of k_selld_union, then those of k_longest
-        GIS_HIP(h, ucount.ensure(sizeof(int) * ((size_t)S + 6)));
+        GIS_HIP(h, ucount.ensure(sizeof(int) * ((size_t)S + 7)));
         GIS_HIP(h, tmp_offs.ensure(sizeof(int) * 32 * (size_t)S));
         GIS_HIP(h, h->ooff.ensure(sizeof(int) * ((size_t)S + 1)));
         GIS_HIP(h, h->dmask.ensure(sizeof(unsigned) * (size_t)N));
         GIS_HIP(h, h->dmask8.ensure((size_t)N));
-        GIS_HIP(h, hipMemsetAsync(ucount.p, 0, sizeof(int) * ((size_t)S + 6), h->stream));
+        GIS_HIP(h, hipMemsetAsync(ucount.p, 0, sizeof(int) * ((size_t)S + 7), h->stream));
         const dim3 gs((unsigned)((S + kBlk / 64 - 1) / (kBlk / 64)));
         hipLaunchKernelGGL(k_selld_union, gs, dim3(kBlk), 0, h->stream, N, S,
                            h->rowptr.as<int>(), h->col.as<int>(), h->soff.as<int>(),
@@ -676,10 +682,10 @@ int build_pattern(gis_context* h, int N, int M, const int* d_la, const int* d_ua
         GIS_HIP(h, hipGetLastError());
         hipLaunchKernelGGL(k_longest, dim3((unsigned)std::min((S + kBlk - 1) / kBlk, 64)),
                            dim3(kBlk), 0, h->stream, S, ucount.as<int>(), h->soff.as<int>(),
-                           ucount.as<int>() + S + 4);
+                           tmp_offs.as<int>(), ucount.as<int>() + S + 4);
         GIS_HIP(h, hipGetLastError());
         GIS_TRY(scan_exclusive(h, ucount.as<int>(), h->ooff.as<int>(), S + 1, tmp, scan_tmp));
-        int n_tab = 0, counts[5] = {0, 0, 0, 0, 0};
+        int n_tab = 0, counts[6] = {0, 0, 0, 0, 0, 0};
         GIS_HIP(h, hipMemcpyAsync(&n_tab, h->ooff.as<int>() + S, sizeof(int),
                                   hipMemcpyDeviceToHost, h->stream));
         GIS_HIP(h, hipMemcpyAsync(counts, ucount.as<int>() + S + 1, sizeof(counts),
@@ -692,6 +698,7 @@ int build_pattern(gis_context* h, int N, int M, const int* d_la, const int* d_ua
         h->lay_untabled_slots = counts[2];
         h->lay_max_table = counts[3];
         h->lay_max_row = counts[4];
+        h->lay_max_offset = counts[5];
         h->n_dslots = 64LL * n_tab;
         GIS_HIP(h, h->doffs.ensure(sizeof(int) * std::max(n_tab, 1)));
         GIS_HIP(h, h->dperm.ensure(sizeof(int) * (size_t)std::max<long long>(h->n_dslots, 1)));
