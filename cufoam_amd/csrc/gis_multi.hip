@@ -78,7 +78,7 @@ __device__ __forceinline__ void sell_multi(const Mat<T>& m, int N, int row0, XOp
                 for (int u = 0; u < kB; ++u) cc[u] = min(max(row + o8[u], 0), last);
 #pragma unroll
                 for (int u = 0; u < kB; ++u) {
-                    const bool on = (mask >> (j + u)) & 1u;
+                    const bool on = slot_bit(mask, j, u);
 #pragma unroll
                     for (int k = 0; k < NR; ++k) {
                         const bool use = on && ((active >> k) & 1u);
