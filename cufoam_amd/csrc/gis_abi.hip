@@ -642,6 +642,16 @@ GIS_API int gis_solve_pcg_device(gis_handle h, int precond, double* d_x, const d
     return pcg_impl(h, precond, d_x, d_b, params, hist, hist_cap, hist_len, true);
 }
 
+GIS_API int gis_get_resident_counts(gis_handle h, gis_resident_counts* out) {
+    if (!h) return GIS_ERR_ARG;
+    if (!out) return fail(h, GIS_ERR_ARG, "get_resident_counts: null output");
+    out->ran = h->res_count[kResRan];
+    out->unfit = h->res_count[kResUnfit];
+    out->late = h->res_count[kResTooLate];
+    out->skipped = h->res_count[kResSkipped];
+    return GIS_OK;
+}
+
 GIS_API int gis_set_slot_fault(gis_handle h, int polls) {
     if (!h) return GIS_ERR_ARG;
     if (polls < 0) return fail(h, GIS_ERR_ARG, "polls must be >= 0");

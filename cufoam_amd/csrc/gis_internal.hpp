@@ -46,6 +46,11 @@ struct DevMem {
     ~DevMem() { release(); }
 };
 
+// Resident solves (gis_resident.hip): the forms, each with its own halo capacity,
+// and what their launches came to (gis_resident_counts).
+enum : int { kResCg = 0, kResBicg = 1, kResBatch = 2, kResForms = 3 };
+enum : int { kResRan = 0, kResUnfit = 1, kResTooLate = 2, kResSkipped = 3, kResCounts = 4 };
+
 // SpMV schedule: how a tile's products are formed.  Every schedule yields
 // bit-identical results (same per-row order), so the choice is pure tuning.
 enum class SpmvKind : int {
@@ -237,7 +242,8 @@ struct gis_context {
     gis::DevMem res_mem;                        // slots and handshake of resident solves
     int n_cu = 0;                               // compute units of the device
     bool sched_pinned = false;                  // gis_set_schedule chose the FP64 kernels
-    bool res_unfit = false;                     // the pattern takes no resident form
+    bool res_unfit[gis::kResForms] = {};        // the pattern's halo does not fit the form
+    long long res_count[gis::kResCounts] = {};  // gis_get_resident_counts
 
     gis::Schedule sched;
     gis::Timer timer;

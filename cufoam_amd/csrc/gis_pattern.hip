@@ -554,7 +554,7 @@ int build_pattern(gis_context* h, int N, int M, const int* d_la, const int* d_ua
         return fail(h, kErrShape,
                     "n_cells must be >= 1 and n_cells + 2*n_faces + n_couples < 2^31");
     h->has_pattern = false;
-    h->res_unfit = false;
+    for (bool& unfit : h->res_unfit) unfit = false;
     h->has_values = h->has_val32 = h->has_valT = h->has_val32T = false;
     if (h->amg) h->amg->clear();
     GIS_HIP(h, h->rowptr.ensure(sizeof(int) * ((size_t)N + 1)));

@@ -852,13 +852,23 @@ std::mutex g_resident[kResDevices];
 // Iterations per launch: the host looks at the state in between.
 constexpr int kResChunk = 2048;
 
+// A launch's verdict (0: it ran) into the handle's counts.
+void count_launch(gis_context* h, int verdict) {
+    ++h->res_count[verdict == 0           ? kResRan
+                   : verdict == kResNoFit ? kResUnfit
+                                          : kResTooLate];
+}
+
 // Launches chunks until the solve is done.  launch(ws) enqueues one.  *ran =
 // false: nothing was done.
 template <class Launch>
-int run_resident(gis_context* h, Launch&& launch, bool* ran) {
+int run_resident(gis_context* h, int form, Launch&& launch, bool* ran) {
     *ran = false;
     std::unique_lock<std::mutex> lock(g_resident[h->device], std::try_to_lock);
-    if (!lock.owns_lock()) return kOK;
+    if (!lock.owns_lock()) {
+        ++h->res_count[kResSkipped];
+        return kOK;
+    }
     const size_t n_slot = (size_t)kResSets * kResSlots;
     GIS_HIP(h, h->res_mem.ensure(sizeof(double) * n_slot + 64));
     double* s = h->res_mem.as<double>();
@@ -870,7 +880,8 @@ int run_resident(gis_context* h, Launch&& launch, bool* ran) {
         GIS_HIP(h, hipGetLastError());
         GIS_TRY(read_state(h));
         const KState& st = *h->st_host;
-        if (st.flag == kResNoFit) h->res_unfit = true;   // the pattern's halo is too large
+        if (st.flag == kResNoFit) h->res_unfit[form] = true;   // the pattern's halo is too large
+        count_launch(h, st.flag);
         if (st.flag != 0 && !*ran) return kOK;
         // a later chunk that could not start is tried again: its r and p are the
         // resident form's
@@ -887,9 +898,10 @@ __global__ void k_res_reset_all(int* sync, int n) {
 
 // TAB form of the pattern; false: it takes no resident form.  The int32 slots
 // serve where some slice has no offset table, or a long one.
-bool res_form(const gis_context* h, bool* tab) {
+bool res_form(const gis_context* h, int form, bool* tab) {
     // iteration timers count the stages' launches; a chosen schedule is a choice of them
-    if (h->sched_pinned || (h->timer.mask & 0x13) || h->res_unfit || h->device >= kResDevices)
+    if (h->sched_pinned || (h->timer.mask & 0x13) || h->res_unfit[form] ||
+        h->device >= kResDevices)
         return false;
     *tab = h->lay_table_slices == h->lay_slices && h->lay_max_table <= kResEntries;
     return *tab || h->lay_max_row <= kResEntries;
@@ -908,12 +920,12 @@ int res_cg_tiles(const gis_context* h) {
 
 bool resident_cg_fits(const gis_context* h) {
     bool tab;
-    return res_form(h, &tab) && res_cg_tiles(h) != 0;
+    return res_form(h, kResCg, &tab) && res_cg_tiles(h) != 0;
 }
 
 bool resident_bicg_fits(const gis_context* h) {
     bool tab;
-    return res_form(h, &tab) && tiles_of(h->N) <= std::min(h->n_cu, kResMaxGrid);
+    return res_form(h, kResBicg, &tab) && tiles_of(h->N) <= std::min(h->n_cu, kResMaxGrid);
 }
 
 int resident_cg(gis_context* h, const Mat<double>& m, double* r, double* p, double* qx, double* x,
@@ -921,9 +933,9 @@ int resident_cg(gis_context* h, const Mat<double>& m, double* r, double* p, doub
     *ran = false;
     bool tab;
     const int rpt = res_cg_tiles(h);
-    if (!res_form(h, &tab) || rpt == 0) return kOK;
+    if (!res_form(h, kResCg, &tab) || rpt == 0) return kOK;
     const dim3 g((unsigned)((tiles_of(h->N) + rpt - 1) / rpt));
-    return run_resident(h, [&](const ResWs& ws) {
+    return run_resident(h, kResCg, [&](const ResWs& ws) {
         const auto go = [&](auto k) {
             hipLaunchKernelGGL(k, g, dim3(kResWG), 0, h->stream, m, h->N, r, p, qx, x, h->st, ws,
                                kResChunk);
@@ -942,9 +954,9 @@ int resident_bicg(gis_context* h, const Mat<double>& m, const Mat<double>& mt, d
                   double* rs, double* p, double* ps, double* qx, double* x, bool* ran) {
     *ran = false;
     bool tab;
-    if (!resident_bicg_fits(h) || !res_form(h, &tab)) return kOK;
+    if (!resident_bicg_fits(h) || !res_form(h, kResBicg, &tab)) return kOK;
     const dim3 g((unsigned)tiles_of(h->N));
-    return run_resident(h, [&](const ResWs& ws) {
+    return run_resident(h, kResBicg, [&](const ResWs& ws) {
         const auto go = [&](auto k) {
             hipLaunchKernelGGL(k, g, dim3(kResWG), 0, h->stream, m, mt, h->N, r, rs, p, ps, qx, x,
                                h->st, ws, kResChunk);
@@ -1003,7 +1015,10 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
         B.res_first = first;
     }
     std::unique_lock<std::mutex> lock(g_resident[h->device], std::try_to_lock);
-    if (!lock.owns_lock()) return kOK;
+    if (!lock.owns_lock()) {
+        ++h->res_count[kResSkipped];
+        return kOK;
+    }
     const int L = (int)B.res_first.size() - 1;
     const size_t n_slot = (size_t)B.res_slots * kResSets * kResSlots;
     GIS_HIP(h, h->res_mem.ensure(sizeof(double) * n_slot + sizeof(int) * 4 * (size_t)L));
@@ -1029,8 +1044,10 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
         GIS_HIP(h, hipMemcpyAsync(verdict.data(), sync, sizeof(int) * 4 * (size_t)L,
                                   hipMemcpyDeviceToHost, h->stream));
         GIS_HIP(h, hipStreamSynchronize(h->stream));
-        for (int l = 0; l < L; ++l)
-            if (verdict[4 * l + 2] == kResNoFit) h->res_unfit = true;
+        for (int l = 0; l < L; ++l) {
+            if (verdict[4 * l + 2] == kResNoFit) h->res_unfit[kResBatch] = true;
+            count_launch(h, verdict[4 * l + 2]);
+        }
         // a system that a chunk left unfinished goes on in its resident form
         bool open = false;
         for (int i = 0; i < S; ++i) open = open || (!B.st_host[i].done && B.st_host[i].k > 0);
@@ -1041,7 +1058,7 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
 
 bool resident_batch_fits(const gis_context* h) {
     bool tab;
-    if (!res_form(h, &tab) || h->lay_max_row > kResEntries) return false;
+    if (!res_form(h, kResBatch, &tab) || h->lay_max_row > kResEntries) return false;
     const BatchInfo& B = h->batch;
     const int n_cu = std::min(h->n_cu, kResMaxGrid);
     int most = 0;

@@ -49,6 +49,10 @@ class _Layout(C.Structure):
                                             "byte_mask_slices", "untabled_slots")]
 
 
+class _ResidentCounts(C.Structure):
+    _fields_ = [(f, C.c_longlong) for f in ("ran", "unfit", "late", "skipped")]
+
+
 class _Perf(C.Structure):
     _fields_ = [("initial_residual", C.c_double), ("final_residual", C.c_double),
                 ("n_iterations", C.c_int), ("status", C.c_int), ("norm_factor", C.c_double)]
@@ -77,6 +81,7 @@ SIGNATURES = {
     "gis_set_coupled_values_device": (_i, [_vp, _vp, _vp, _vp, _vp]),
     "gis_get_size": (_i, [_vp, _ip, _llp]),
     "gis_get_layout": (_i, [_vp, C.POINTER(_Layout)]),
+    "gis_get_resident_counts": (_i, [_vp, C.POINTER(_ResidentCounts)]),
     "gis_get_csr": (_i, [_vp, _vp, _vp, _vp]),
     "gis_get_csr_transpose": (_i, [_vp, _vp, _vp, _vp]),
     "gis_spmv_device": (_i, [_vp, _vp, _vp]),
@@ -403,6 +408,12 @@ class Gis:
         lay = _Layout()
         self._check(self._L.gis_get_layout(self._h, C.byref(lay)), "get_layout")
         return {f: getattr(lay, f) for f, _ in _Layout._fields_}
+
+    def resident_counts(self) -> dict:
+        """What the handle's resident launches came to (gis_resident_counts)."""
+        c = _ResidentCounts()
+        self._check(self._L.gis_get_resident_counts(self._h, C.byref(c)), "get_resident_counts")
+        return {f: getattr(c, f) for f, _ in _ResidentCounts._fields_}
 
     def set_symmetric_storage(self, enable: bool = True):
         """Switch the symmetric storage of the offset-table schedule on or off

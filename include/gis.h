@@ -184,6 +184,19 @@ typedef struct gis_schedule {
 GIS_API int gis_set_schedule(gis_handle h, const gis_schedule *s);
 GIS_API int gis_get_schedule(gis_handle h, gis_schedule *s);
 
+/* ---- resident solves (no counterpart in the reference): CG, BiCG and batched CG
+ * of systems that fit the chip run as one launch per solve, or per 2048 iterations,
+ * whose workgroups start together or not at all; otherwise the solve runs one
+ * launch per stage.  Counts since gis_create. ---- */
+typedef struct {
+    long long ran;      /* launches that ran */
+    long long unfit;    /* launches that gave up: too many rows of other workgroups are
+                           referred to (the form is not tried again for the pattern) */
+    long long late;     /* launches that gave up: not all workgroups came to run */
+    long long skipped;  /* solves that started none: another resident solve was running */
+} gis_resident_counts;
+GIS_API int gis_get_resident_counts(gis_handle h, gis_resident_counts *out);
+
 /* ---- autotuner: times every (SpMV schedule x direction form x tiles per
  * workgroup) candidate on the
  * handle's matrix with `iterations` solver iterations per run (<= 0: 24) and

@@ -20,6 +20,13 @@ def stages(g, f):
     return f(g)
 
 
+def counted(g, f):
+    """f(g) and how much each of the handle's resident counts grew."""
+    before = g.resident_counts()
+    out = f(g)
+    return out, {k: v - before[k] for k, v in g.resident_counts().items() if v != before[k]}
+
+
 def banded(n, width, seed):
     """n cells on a line, each coupled to the next and to the one `width` on."""
     rng = np.random.default_rng(seed)
@@ -196,3 +203,24 @@ def test_batch_mixed_fit(gpu):
         assert it[i] == ref.iterations
         np.testing.assert_array_equal(x[off:off + s.n_cells], ref.x)
         off += s.n_cells
+
+
+@pytest.mark.parametrize("first", ["CG", "BiCG"])
+def test_one_form_that_does_not_fit_leaves_the_other(gpu, first):
+    """About 6000 halo rows a workgroup: past BiCG's 4096, within CG's 8192.  The
+    route of either does not depend on which ran first."""
+    s = mesh.laplacian(40, seed=3, shift=1e-2)
+    s = mesh.renumber(s, np.random.default_rng(1).permutation(s.n_cells))
+    gpu.set_system(s)
+    order = ["CG", "BiCG"] if first == "CG" else ["BiCG", "CG"]
+    for rep in range(2):
+        for method in order:
+            (x, hist, _), grew = counted(
+                gpu, lambda g: g.solve(method, s.b, s.x0, error=0.0, max_steps=20))
+            if method == "CG":
+                assert grew == {"ran": 1}
+            else:
+                assert grew == ({"unfit": 1} if rep == 0 else {})
+            ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, 0.0, 20)
+            np.testing.assert_array_equal(hist, ref.hist)
+            np.testing.assert_array_equal(x, ref.x)
