@@ -652,6 +652,14 @@ GIS_API int gis_get_resident_counts(gis_handle h, gis_resident_counts* out) {
     return GIS_OK;
 }
 
+GIS_API int gis_set_late_launches(gis_handle h, int after, int count) {
+    if (!h) return GIS_ERR_ARG;
+    if (after < 0 || count < 0) return fail(h, GIS_ERR_ARG, "late launches: need counts >= 0");
+    h->late_after = after;
+    h->late_n = count;
+    return GIS_OK;
+}
+
 GIS_API int gis_set_slot_fault(gis_handle h, int polls) {
     if (!h) return GIS_ERR_ARG;
     if (polls < 0) return fail(h, GIS_ERR_ARG, "polls must be >= 0");

@@ -244,6 +244,8 @@ struct gis_context {
     bool sched_pinned = false;                  // gis_set_schedule chose the FP64 kernels
     bool res_unfit[gis::kResForms] = {};        // the pattern's halo does not fit the form
     long long res_count[gis::kResCounts] = {};  // gis_get_resident_counts
+    int res_skip = 0, res_backoff = 0;          // solves held back after a late grid
+    int late_after = 0, late_n = 0;             // gis_set_late_launches (failure-path tests)
 
     gis::Schedule sched;
     gis::Timer timer;

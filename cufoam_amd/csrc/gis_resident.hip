@@ -22,7 +22,8 @@
 // resident.  A launch therefore starts with a handshake: it goes ahead only
 // once every workgroup has arrived, and gives up (having changed nothing) when
 // that takes too long, for instance because another program's kernel holds
-// compute units.  The caller then runs the launch-per-stage loop.
+// compute units.  The caller then runs the launch-per-stage loop, and the next
+// solves go there without waiting.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -839,8 +840,10 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
     }
 }
 
-__global__ void k_res_reset(ResWs ws, KState* st) {
-    if (threadIdx.x < 2) ws.sync[threadIdx.x] = 0;
+// verdict: kResWait, or kResLate for a launch that is to find its grid late
+__global__ void k_res_reset(ResWs ws, KState* st, int verdict) {
+    if (threadIdx.x == 0) ws.sync[0] = 0;
+    if (threadIdx.x == 1) ws.sync[1] = verdict;
     if (threadIdx.x == 2) st->flag = 0;
 }
 
@@ -851,6 +854,47 @@ std::mutex g_resident[kResDevices];
 
 // Iterations per launch: the host looks at the state in between.
 constexpr int kResChunk = 2048;
+
+// How long a launch waits for its grid.  A solve that is under way has nothing
+// else to do, so its later launches wait up to 16 times as long, and are tried
+// again until about 80 s have gone.
+constexpr double kResPatience = 5e-3;
+constexpr int kResRetries = 1000;
+
+// After a launch whose grid came late (another program's kernels hold compute
+// units), the next 1, 3, 7, .. 63 solves of the handle go stage by stage without
+// waiting for theirs: at most one solve in 64 then pays the 5 ms.  A launch that
+// runs ends it.
+constexpr int kResMaxBackoff = 63;
+
+bool held_back(gis_context* h) {
+    if (h->res_skip == 0) return false;
+    --h->res_skip;
+    ++h->res_count[kResSkipped];
+    return true;
+}
+
+void hold_back_next(gis_context* h, bool late) {
+    h->res_backoff = late ? std::min(2 * h->res_backoff + 1, kResMaxBackoff) : 0;
+    h->res_skip = h->res_backoff;
+}
+
+long long patience_ticks(const gis_context* h, int late) {
+    const double tick = h->wall_tick > 0.0 ? h->wall_tick : 1e-8;
+    return (long long)(kResPatience / tick) << std::min(late, 4);
+}
+
+// gis_set_late_launches: which of the next n launches find their grid late
+struct LateLaunches {
+    int first, end;
+};
+
+LateLaunches late_launches(gis_context* h, int n) {
+    const int first = std::min(h->late_after, n), end = first + std::min(h->late_n, n - first);
+    h->late_after -= first;
+    h->late_n -= end - first;
+    return {first, end};
+}
 
 // A launch's verdict (0: it ran) into the handle's counts.
 void count_launch(gis_context* h, int verdict) {
@@ -864,6 +908,7 @@ void count_launch(gis_context* h, int verdict) {
 template <class Launch>
 int run_resident(gis_context* h, int form, Launch&& launch, bool* ran) {
     *ran = false;
+    if (held_back(h)) return kOK;
     std::unique_lock<std::mutex> lock(g_resident[h->device], std::try_to_lock);
     if (!lock.owns_lock()) {
         ++h->res_count[kResSkipped];
@@ -872,28 +917,32 @@ int run_resident(gis_context* h, int form, Launch&& launch, bool* ran) {
     const size_t n_slot = (size_t)kResSets * kResSlots;
     GIS_HIP(h, h->res_mem.ensure(sizeof(double) * n_slot + 64));
     double* s = h->res_mem.as<double>();
-    const double tick = h->wall_tick > 0.0 ? h->wall_tick : 1e-8;
-    const ResWs ws{s, reinterpret_cast<int*>(s + n_slot), (long long)(5e-3 / tick)};
     for (int late = 0;;) {
-        hipLaunchKernelGGL(k_res_reset, dim3(1), dim3(64), 0, h->stream, ws, h->st);
+        const ResWs ws{s, reinterpret_cast<int*>(s + n_slot), patience_ticks(h, late)};
+        const LateLaunches f = late_launches(h, 1);
+        hipLaunchKernelGGL(k_res_reset, dim3(1), dim3(64), 0, h->stream, ws, h->st,
+                           f.first < f.end ? kResLate : kResWait);
         launch(ws);
         GIS_HIP(h, hipGetLastError());
         GIS_TRY(read_state(h));
         const KState& st = *h->st_host;
         if (st.flag == kResNoFit) h->res_unfit[form] = true;   // the pattern's halo is too large
         count_launch(h, st.flag);
+        if (!*ran) hold_back_next(h, st.flag == kResLate);
         if (st.flag != 0 && !*ran) return kOK;
         // a later chunk that could not start is tried again: its r and p are the
         // resident form's
-        if (st.flag != 0 && ++late > 1000)
+        if (st.flag != 0 && ++late > kResRetries)
             return fail(h, kErrSync, "the solve's grid could not be made resident again");
         *ran = true;
         if (st.done) return kOK;
     }
 }
 
-__global__ void k_res_reset_all(int* sync, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) sync[i] = 0;
+// 4 words a launch; launches [late0, late1) are to find their grid late
+__global__ void k_res_reset_all(int* sync, int n, int late0, int late1) {
+    for (int i = threadIdx.x; i < 4 * n; i += blockDim.x)
+        sync[i] = i % 4 == 1 && i / 4 >= late0 && i / 4 < late1 ? kResLate : 0;
 }
 
 // TAB form of the pattern; false: it takes no resident form.  The int32 slots
@@ -1014,6 +1063,7 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
         B.res_slots = slots;
         B.res_first = first;
     }
+    if (held_back(h)) return kOK;
     std::unique_lock<std::mutex> lock(g_resident[h->device], std::try_to_lock);
     if (!lock.owns_lock()) {
         ++h->res_count[kResSkipped];
@@ -1024,12 +1074,14 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
     GIS_HIP(h, h->res_mem.ensure(sizeof(double) * n_slot + sizeof(int) * 4 * (size_t)L));
     double* slot = h->res_mem.as<double>();
     int* sync = reinterpret_cast<int*>(slot + n_slot);
-    const double tick = h->wall_tick > 0.0 ? h->wall_tick : 1e-8;
     std::vector<int> verdict(4 * (size_t)L);
-    for (int late = 0; late <= 1000; ++late) {
-        hipLaunchKernelGGL(k_res_reset_all, dim3(1), dim3(kWG), 0, h->stream, sync, 4 * L);
+    bool first = true;
+    for (int late = 0;;) {
+        const LateLaunches f = late_launches(h, L);
+        hipLaunchKernelGGL(k_res_reset_all, dim3(1), dim3(kWG), 0, h->stream, sync, L, f.first,
+                           f.end);
         for (int l = 0; l < L; ++l) {
-            const ResWs ws{slot, sync + 4 * l, (long long)(5e-3 / tick)};
+            const ResWs ws{slot, sync + 4 * l, patience_ticks(h, late)};
             const dim3 g((unsigned)(B.res_first[l + 1] - B.res_first[l]));
             const auto go = [&](auto k) {
                 hipLaunchKernelGGL(k, g, dim3(kResWG), 0, h->stream, m, (size_t)h->N, r, p, qx, x,
@@ -1044,16 +1096,21 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
         GIS_HIP(h, hipMemcpyAsync(verdict.data(), sync, sizeof(int) * 4 * (size_t)L,
                                   hipMemcpyDeviceToHost, h->stream));
         GIS_HIP(h, hipStreamSynchronize(h->stream));
+        bool any_late = false;
         for (int l = 0; l < L; ++l) {
             if (verdict[4 * l + 2] == kResNoFit) h->res_unfit[kResBatch] = true;
             count_launch(h, verdict[4 * l + 2]);
+            any_late = any_late || verdict[4 * l + 2] == kResLate;
         }
+        if (first) hold_back_next(h, any_late);
+        first = false;
         // a system that a chunk left unfinished goes on in its resident form
         bool open = false;
         for (int i = 0; i < S; ++i) open = open || (!B.st_host[i].done && B.st_host[i].k > 0);
         if (!open) return kOK;
+        if (any_late && ++late > kResRetries)
+            return fail(h, kErrSync, "the batch's grid could not be made resident again");
     }
-    return fail(h, kErrSync, "the batch's grid could not be made resident again");
 }
 
 bool resident_batch_fits(const gis_context* h) {

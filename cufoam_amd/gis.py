@@ -110,6 +110,7 @@ SIGNATURES = {
     "gis_foam_solve_pbicg": (_i, [_vp, _i, _vp, _vp, _d, _d, _ll, _ll, C.POINTER(_Perf)]),
     "gis_set_gamg": (_i, [_vp, _d, _i, _d]),
     "gis_set_slot_fault": (_i, [_vp, _i]),
+    "gis_set_late_launches": (_i, [_vp, _i, _i]),
     "gis_set_timing_sample": (_i, [_vp, _i]),
     "gis_set_symmetric_storage": (_i, [_vp, _i]),
     "gis_get_symmetric_storage": (_i, [_vp, _ip, C.POINTER(C.c_longlong)]),
@@ -605,6 +606,12 @@ class Gis:
         self._check(st, f"solve_pbicg({precond})")
         self.last_iterations = max(hl.value - 1, 0)
         return x, hist[:min(hl.value, hist_cap)].copy(), st
+
+    def set_late_launches(self, after: int, count: int):
+        """Failure-path tests only: `count` resident launches, after `after` more of
+        them, find their grid late (gis_set_late_launches)."""
+        self._check(self._L.gis_set_late_launches(self._h, int(after), int(count)),
+                    "set_late_launches")
 
     def set_slot_fault(self, polls: int = 0):
         """Failure-path tests only: polls > 0 makes every device reduction give up

@@ -193,7 +193,8 @@ typedef struct {
     long long unfit;    /* launches that gave up: too many rows of other workgroups are
                            referred to (the form is not tried again for the pattern) */
     long long late;     /* launches that gave up: not all workgroups came to run */
-    long long skipped;  /* solves that started none: another resident solve was running */
+    long long skipped;  /* solves that started none: another resident solve was running,
+                           or (for 1, 3, 7, .. 63 solves) the last launch was late */
 } gis_resident_counts;
 GIS_API int gis_get_resident_counts(gis_handle h, gis_resident_counts *out);
 
@@ -361,6 +362,10 @@ GIS_API int gis_set_gamg(gis_handle h, double omega, int nu, double cscale);
  * stops with GIS_ERR_SYNC; polls = 0 restores normal operation.  The kernels
  * still exit normally.  Applies to solves started after the call. ---- */
 GIS_API int gis_set_slot_fault(gis_handle h, int polls);
+/* Failure-path tests only: after `after` more resident launches of the handle,
+ * `count` of them find their workgroups not all there in time and give up (the
+ * kernels exit normally); a launch of one workgroup waits for nobody. */
+GIS_API int gis_set_late_launches(gis_handle h, int after, int count);
 /* The hierarchy (built if needed): level count, then one level's sizes,
  * aggregation map (cell -> next-level cell; levels below the last) and LDU
  * matrix (any output pointer may be NULL). */

@@ -224,3 +224,89 @@ def test_one_form_that_does_not_fit_leaves_the_other(gpu, first):
             ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, 0.0, 20)
             np.testing.assert_array_equal(hist, ref.hist)
             np.testing.assert_array_equal(x, ref.x)
+
+
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_late_grid_falls_back_and_holds_back(gpu, method):
+    """A first launch that finds its grid late leaves the solve to the stages; the
+    next 1, then 3 solves do not wait for theirs; a launch that runs ends that."""
+    s = mesh.laplacian(14, seed=9, shift=1e-2, symmetric=method == "CG")
+    gpu.set_system(s)
+    ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, 1e-9, 400)
+
+    def solve(g):
+        x, hist, _ = g.solve(method, s.b, s.x0, error=1e-9, max_steps=400)
+        np.testing.assert_array_equal(hist, ref.hist)
+        np.testing.assert_array_equal(x, ref.x)
+    gpu.set_late_launches(0, 2)
+    want = [{"late": 1}, {"skipped": 1}, {"late": 1}] + [{"skipped": 1}] * 3 + [{"ran": 1}] * 2
+    for grew in want:
+        assert counted(gpu, solve)[1] == grew
+
+
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_late_grid_between_launches(gpu, method):
+    """A launch in the middle of a solve that finds its grid late is tried again."""
+    s = mesh.laplacian(14, seed=9, shift=1e-3, symmetric=method == "CG")
+    gpu.set_system(s)
+    ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, -1.0, 4100)
+    gpu.set_late_launches(1, 2)
+    (x, hist, _), grew = counted(
+        gpu, lambda g: g.solve(method, s.b, s.x0, error=-1.0, max_steps=4100))
+    assert grew == {"ran": -(-(len(hist) - 1) // 2048), "late": 2} and grew["ran"] > 1
+    np.testing.assert_array_equal(hist, ref.hist)
+    np.testing.assert_array_equal(x, ref.x)
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+@pytest.mark.parametrize("after,count", [(0, 1), (1, 1), (0, 9)])
+def test_late_batch(gpu, use_graph, after, count):
+    """Systems whose launch finds its grid late are left to the stage loop, beside
+    those that ran."""
+    systems = [mesh.laplacian(n, seed=60 + i, shift=1e-2) for i, n in enumerate([40, 64, 3, 65, 30])]
+    err = np.array([1e-6 * np.linalg.norm(s.b) for s in systems])
+    b = np.concatenate([s.b for s in systems])
+    gpu.batch_set_systems(systems)
+
+    def run(g):
+        return g.batch_solve(b, None, err, 300, use_graph=use_graph)
+    want, grew = counted(gpu, run)
+    assert set(grew) == {"ran"} and grew["ran"] >= 2
+    gpu.set_late_launches(after, count)
+    got, late = counted(gpu, run)
+    gpu.set_late_launches(0, 0)
+    n = min(count, grew["ran"] - after)
+    assert late == {k: v for k, v in (("late", n), ("ran", grew["ran"] - n)) if v}
+    held, grew = counted(gpu, run)
+    assert grew == {"skipped": 1}
+    for u, v, w in zip(want, got, held):
+        np.testing.assert_array_equal(u, v)
+        np.testing.assert_array_equal(u, w)
+
+
+def test_two_threads(gpu):
+    """Two handles in two threads: while one's resident solve runs, the other's go
+    stage by stage, with the same bits."""
+    import threading
+
+    from cufoam_amd.gis import Gis
+    s = mesh.laplacian(48, seed=12, shift=1e-3)
+    ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, -1.0, 60)
+    done = threading.Event()
+
+    def long_solves():
+        with Gis(0) as g:
+            g.set_system(s)
+            for _ in range(4):
+                g.solve("CG", s.b, s.x0, error=-1.0, max_steps=8000, hist_cap=1)
+        done.set()
+    gpu.set_system(s)
+    before = gpu.resident_counts()
+    t = threading.Thread(target=long_solves)
+    t.start()
+    while not done.is_set():
+        x, hist, _ = gpu.solve("CG", s.b, s.x0, error=-1.0, max_steps=60)
+        np.testing.assert_array_equal(hist, ref.hist)
+        np.testing.assert_array_equal(x, ref.x)
+    t.join()
+    assert gpu.resident_counts()["skipped"] > before["skipped"]
