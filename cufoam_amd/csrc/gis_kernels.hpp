@@ -454,10 +454,11 @@ int run_blocks(gis_context* h, long long max_steps, Iter&& launch_iteration,
 
 int prepare_solve(gis_context* h, const SolveArgs& a, int nvec);
 // CG with the matrix m, BiCG with m and its transpose mt; the state is left on the
-// device, with a mirror in h->st_host
+// device, with a mirror in h->st_host.  resident given: only as a resident solve;
+// *resident = false where that did not start (x unchanged).
 int solve_cg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, double* x,
-                const double* b);
+                const double* b, bool* resident = nullptr);
 int solve_bicg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, const Mat<double>& mt,
-                  double* x, const double* b);
+                  double* x, const double* b, bool* resident = nullptr);
 
 }  // namespace gis

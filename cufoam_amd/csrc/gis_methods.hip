@@ -698,7 +698,7 @@ int solve_bicg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
 }  // namespace
 
 int solve_bicg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, const Mat<double>& mt,
-                  double* x, const double* b) {
+                  double* x, const double* b, bool* resident) {
     GIS_TRY(prepare_solve(h, a, resident_bicg_fits(h) ? 4 + 2 * kResQ : 6));
     const int N = h->N;
     double* r = h->vec.as<double>();
@@ -708,9 +708,10 @@ int solve_bicg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, cons
     double* ps = r + 4 * (size_t)N;
     double* q = r + 5 * (size_t)N;
     GIS_TRY(launch_setup(h, m, b, x, nullptr, r, rs, 1));
-    bool resident = false;   // p in pb0, p* in pb1, the exchanged q and q* from ps on
-    GIS_TRY(resident_bicg(h, m, mt, r, rs, pb0, pb1, ps, x, &resident));
-    if (resident) return kOK;
+    bool ran = false;   // p in pb0, p* in pb1, the exchanged q and q* from ps on
+    GIS_TRY(resident_bicg(h, m, mt, r, rs, pb0, pb1, ps, x, &ran));
+    if (resident) *resident = ran;
+    if (ran || resident) return kOK;
     const dim3 g = tiles_grid(N);
     GIS_SPMV_DISPATCH(h->sched.spmv64, P, {
         GIS_TRY(run_blocks(h, iteration_budget(h), [&]() -> int {

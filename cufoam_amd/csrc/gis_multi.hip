@@ -775,29 +775,36 @@ int solve_multi_mixed_nr(gis_context* h, int method, const MultiMixedArgs& a, do
     return kOK;
 }
 
-// Columns solved one after another, each as a single-RHS solve (the bits of its
-// column in the SpMM solve).
+// Column k's outcome from its state; returns its status.
+int column_outcome(const KState& s, int k, int* iters, double* norm0, double* normf, int* status) {
+    int sk = s.status;
+    if (sk == kOK && !(s.norm == s.norm)) sk = kNaN;
+    if (iters) iters[k] = s.k;
+    if (norm0) norm0[k] = s.norm0;
+    if (normf) normf[k] = s.norm;
+    if (status) status[k] = sk;
+    return sk;
+}
+
+// The first columns, one after another, each as a resident single-RHS solve (the
+// bits of its column in the SpMM solve), up to one whose launch does not start:
+// *solved of them, their worst outcome in *worst.
 int solve_columns(gis_context* h, int method, int nrhs, bool transpose, const SolveArgs& a,
                   double* X, const double* B, int* iters, double* norm0, double* normf,
-                  int* status) {
+                  int* status, int* solved, int* worst) {
     const Mat<double> mA = transpose ? mat64T(h) : mat64(h);
     const Mat<double> mAt = transpose ? mat64(h) : mat64T(h);
     const size_t n = (size_t)h->N;
-    int worst = kOK;
-    for (int k = 0; k < nrhs; ++k) {
-        GIS_TRY(method == 0 ? solve_cg_on(h, a, mA, X + k * n, B + k * n)
-                            : solve_bicg_on(h, a, mA, mAt, X + k * n, B + k * n));
+    for (*solved = 0; *solved < nrhs; ++*solved) {
+        const int k = *solved;
+        bool ran = false;
+        GIS_TRY(method == 0 ? solve_cg_on(h, a, mA, X + k * n, B + k * n, &ran)
+                            : solve_bicg_on(h, a, mA, mAt, X + k * n, B + k * n, &ran));
+        if (!ran) break;
         GIS_TRY(read_state(h));
-        const KState& s = *h->st_host;
-        int sk = s.status;
-        if (sk == kOK && !(s.norm == s.norm)) sk = kNaN;
-        if (iters) iters[k] = s.k;
-        if (norm0) norm0[k] = s.norm0;
-        if (normf) normf[k] = s.norm;
-        if (status) status[k] = sk;
-        worst = std::max(worst, sk);
+        *worst = std::max(*worst, column_outcome(*h->st_host, k, iters, norm0, normf, status));
     }
-    return worst;
+    return kOK;
 }
 
 // Columns up to which that is the faster form (one, two, three and five columns
@@ -825,27 +832,27 @@ int device_solve_multi(gis_context* h, int method, int nrhs, bool transpose, con
     if (nrhs < 1 || nrhs > kMaxRhs) return fail(h, kErrArg, "nrhs must be in 1..8");
     if (method != 0 && method != 1) return fail(h, kErrArg, "multi-RHS solves support CG and BiCG");
     GIS_TRY(ensure_valT(h));
+    int worst = kOK, first = 0;
     // a few columns of a system that fits the chip: one resident solve each
-    if (nrhs <= kResColumns && (method == 0 ? resident_cg_fits(h) : resident_bicg_fits(h)))
-        return solve_columns(h, method, nrhs, transpose, a, X, B, iters, norm0, normf, status);
+    if (nrhs <= kResColumns && (method == 0 ? resident_cg_fits(h) : resident_bicg_fits(h))) {
+        GIS_TRY(solve_columns(h, method, nrhs, transpose, a, X, B, iters, norm0, normf, status,
+                              &first, &worst));
+        if (first == nrhs) return worst;
+    }
+    // the others together
+    const int left = nrhs - first;
+    const size_t skip = (size_t)first * h->N;
     MultiBufs mb;
-    GIS_TRY(multi_prepare(h, nrhs, a, sizeof(double) * (size_t)h->N * 6 * nrhs, mb));
+    GIS_TRY(multi_prepare(h, left, a, sizeof(double) * (size_t)h->N * 6 * left, mb));
     int st = kOK;
-    GIS_NR_DISPATCH(nrhs, NRC, st = solve_multi_nr<NRC>(h, method, transpose, a, X, B, mb));
+    GIS_NR_DISPATCH(left, NRC,
+                    st = solve_multi_nr<NRC>(h, method, transpose, a, X + skip, B + skip, mb));
     if (st != kOK) return st;
     bool done = false;
-    GIS_TRY(multi_read(h, nrhs, mb, &done));
-    int worst = kOK;
-    for (int k = 0; k < nrhs; ++k) {
-        const KState& s = mb.host[k];
-        int sk = s.status;
-        if (sk == kOK && !(s.norm == s.norm)) sk = kNaN;
-        if (iters) iters[k] = s.k;
-        if (norm0) norm0[k] = s.norm0;
-        if (normf) normf[k] = s.norm;
-        if (status) status[k] = sk;
-        worst = std::max(worst, sk);
-    }
+    GIS_TRY(multi_read(h, left, mb, &done));
+    for (int k = 0; k < left; ++k)
+        worst = std::max(worst, column_outcome(mb.host[k], first + k, iters, norm0, normf,
+                                               status));
     return worst;
 }
 

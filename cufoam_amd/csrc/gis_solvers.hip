@@ -513,7 +513,7 @@ int solve_cg(gis_context* h, const SolveArgs& a, double* x, const double* b) {
 }
 
 int solve_cg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, double* x,
-                const double* b) {
+                const double* b, bool* resident) {
     GIS_TRY(prepare_solve(h, a, resident_cg_fits(h) ? 2 + kResQ : 4));
     const int N = h->N;
     double* r = h->vec.as<double>();
@@ -525,9 +525,10 @@ int solve_cg_on(gis_context* h, const SolveArgs& a, const Mat<double>& m, double
         hipLaunchKernelGGL((k_setup<P>), g, dim3(kWG), 0, h->stream, m, N, b, x, nullptr, r,
                            nullptr, h->st, h->red, 0);
         GIS_HIP(h, hipGetLastError());
-        bool resident = false;   // p in pb0, the exchanged q from pb1 on
-        GIS_TRY(resident_cg(h, m, r, pb0, pb1, x, &resident));
-        if (resident) return kOK;
+        bool ran = false;   // p in pb0, the exchanged q from pb1 on
+        GIS_TRY(resident_cg(h, m, r, pb0, pb1, x, &ran));
+        if (resident) *resident = ran;
+        if (ran || resident) return kOK;
         const bool split = h->sched.fp64_direction != 0;
         GIS_COARSEN_DISPATCH(h->sched.coarsen64, CC, {
             const dim3 gc = super_grid(N, CC);

@@ -20,6 +20,14 @@ def stages(g, f):
     return f(g)
 
 
+@pytest.fixture
+def fresh(gpu):
+    """A handle of the test's own: no solve of it is held back."""
+    from cufoam_amd.gis import Gis
+    with Gis(0) as g:
+        yield g
+
+
 def counted(g, f):
     """f(g) and how much each of the handle's resident counts grew."""
     before = g.resident_counts()
@@ -227,32 +235,32 @@ def test_one_form_that_does_not_fit_leaves_the_other(gpu, first):
 
 
 @pytest.mark.parametrize("method", ["CG", "BiCG"])
-def test_late_grid_falls_back_and_holds_back(gpu, method):
+def test_late_grid_falls_back_and_holds_back(fresh, method):
     """A first launch that finds its grid late leaves the solve to the stages; the
     next 1, then 3 solves do not wait for theirs; a launch that runs ends that."""
     s = mesh.laplacian(14, seed=9, shift=1e-2, symmetric=method == "CG")
-    gpu.set_system(s)
+    fresh.set_system(s)
     ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, 1e-9, 400)
 
     def solve(g):
         x, hist, _ = g.solve(method, s.b, s.x0, error=1e-9, max_steps=400)
         np.testing.assert_array_equal(hist, ref.hist)
         np.testing.assert_array_equal(x, ref.x)
-    gpu.set_late_launches(0, 2)
+    fresh.set_late_launches(0, 2)
     want = [{"late": 1}, {"skipped": 1}, {"late": 1}] + [{"skipped": 1}] * 3 + [{"ran": 1}] * 2
     for grew in want:
-        assert counted(gpu, solve)[1] == grew
+        assert counted(fresh, solve)[1] == grew
 
 
 @pytest.mark.parametrize("method", ["CG", "BiCG"])
-def test_late_grid_between_launches(gpu, method):
+def test_late_grid_between_launches(fresh, method):
     """A launch in the middle of a solve that finds its grid late is tried again."""
     s = mesh.laplacian(14, seed=9, shift=1e-3, symmetric=method == "CG")
-    gpu.set_system(s)
+    fresh.set_system(s)
     ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, -1.0, 4100)
-    gpu.set_late_launches(1, 2)
+    fresh.set_late_launches(1, 2)
     (x, hist, _), grew = counted(
-        gpu, lambda g: g.solve(method, s.b, s.x0, error=-1.0, max_steps=4100))
+        fresh, lambda g: g.solve(method, s.b, s.x0, error=-1.0, max_steps=4100))
     assert grew == {"ran": -(-(len(hist) - 1) // 2048), "late": 2} and grew["ran"] > 1
     np.testing.assert_array_equal(hist, ref.hist)
     np.testing.assert_array_equal(x, ref.x)
@@ -260,24 +268,24 @@ def test_late_grid_between_launches(gpu, method):
 
 @pytest.mark.parametrize("use_graph", [False, True])
 @pytest.mark.parametrize("after,count", [(0, 1), (1, 1), (0, 9)])
-def test_late_batch(gpu, use_graph, after, count):
+def test_late_batch(fresh, use_graph, after, count):
     """Systems whose launch finds its grid late are left to the stage loop, beside
     those that ran."""
     systems = [mesh.laplacian(n, seed=60 + i, shift=1e-2) for i, n in enumerate([40, 64, 3, 65, 30])]
     err = np.array([1e-6 * np.linalg.norm(s.b) for s in systems])
     b = np.concatenate([s.b for s in systems])
-    gpu.batch_set_systems(systems)
+    fresh.batch_set_systems(systems)
 
     def run(g):
         return g.batch_solve(b, None, err, 300, use_graph=use_graph)
-    want, grew = counted(gpu, run)
+    want, grew = counted(fresh, run)
     assert set(grew) == {"ran"} and grew["ran"] >= 2
-    gpu.set_late_launches(after, count)
-    got, late = counted(gpu, run)
-    gpu.set_late_launches(0, 0)
+    fresh.set_late_launches(after, count)
+    got, late = counted(fresh, run)
+    fresh.set_late_launches(0, 0)
     n = min(count, grew["ran"] - after)
     assert late == {k: v for k, v in (("late", n), ("ran", grew["ran"] - n)) if v}
-    held, grew = counted(gpu, run)
+    held, grew = counted(fresh, run)
     assert grew == {"skipped": 1}
     for u, v, w in zip(want, got, held):
         np.testing.assert_array_equal(u, v)
@@ -310,3 +318,41 @@ def test_two_threads(gpu):
         np.testing.assert_array_equal(x, ref.x)
     t.join()
     assert gpu.resident_counts()["skipped"] > before["skipped"]
+
+
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+@pytest.mark.parametrize("after", [0, 1, 2])
+def test_columns_that_do_not_start_go_together(fresh, method, after):
+    """From the first column whose launch finds its grid late, the columns are one
+    SpMM solve: none of them tries a launch of its own."""
+    s = mesh.laplacian(20, seed=4, shift=0.1, symmetric=method == "CG")
+    fresh.set_system(s)
+    A = O.ldu2csr(s)
+    At = O.transpose(A)
+    B = np.random.default_rng(2).uniform(-1, 1, (3, s.n_cells))
+    fresh.set_late_launches(after, 1)
+    (X, it, nf, st), grew = counted(
+        fresh, lambda g: g.solve_multi(method, B, None, error=1e-8, max_steps=300))
+    assert grew == {k: v for k, v in (("ran", after), ("late", 1)) if v}
+    for k in range(3):
+        ref = O.solve(method, A, B[k], np.zeros(s.n_cells), 1e-8, 300, At=At)
+        assert it[k] == ref.iterations and nf[k] == ref.hist[-1]
+        np.testing.assert_array_equal(X[k], ref.x)
+
+
+def test_columns_that_do_not_fit_go_together(gpu):
+    """A halo too large for BiCG: the first column gives up, then all are one solve."""
+    s = mesh.laplacian(40, seed=3, shift=0.1, symmetric=False)
+    s = mesh.renumber(s, np.random.default_rng(1).permutation(s.n_cells))
+    gpu.set_system(s)
+    A = O.ldu2csr(s)
+    At = O.transpose(A)
+    B = np.random.default_rng(2).uniform(-1, 1, (2, s.n_cells))
+    for want in ({"unfit": 1}, {}):
+        (X, it, nf, st), grew = counted(
+            gpu, lambda g: g.solve_multi("BiCG", B, None, error=0.0, max_steps=40))
+        assert grew == want
+        for k in range(2):
+            ref = O.solve("BiCG", A, B[k], np.zeros(s.n_cells), 0.0, 40, At=At)
+            assert it[k] == ref.iterations and nf[k] == ref.hist[-1]
+            np.testing.assert_array_equal(X[k], ref.x)
