@@ -404,6 +404,12 @@ int device_sddmm_fold(gis_context* h, int nrhs, const double* Lam, const double*
 // launches; else the solve is over, x complete.  p, ps and qx (kResQ vectors per
 // exchanged one) are workspace.
 constexpr int kResQ = 3;
+// Steps from which a resident solve is the faster one: its launch sets up the halo
+// and waits for its grid first (stages / resident, us a solve of 1, 2, 3 and 5 steps:
+// CG 16^3 97 / 99, 109 / 103, 125 / 112, 165 / 124; 64^3 104 / 122, 122 / 128,
+// 142 / 141, 186 / 159; 80^3 113 / 141, 134 / 151, 159 / 164, 217 / 188; BiCG 64^3
+// 112 / 129, 133 / 143, 160 / 161, 213 / 187).
+constexpr int kResMinSteps = 3;
 template <typename T>
 struct Mat;
 bool resident_cg_fits(const gis_context* h);

@@ -812,6 +812,16 @@ int solve_columns(gis_context* h, int method, int nrhs, bool transpose, const So
 // 1.0x at 63^3 renumbered; BiCG the same within 5%; faster still below).
 constexpr int kResColumns = 3;
 
+// A solve capped at few steps stays one SpMM solve: each column's own set-up, launch
+// and read of its state cost more than the steps save (SpMM / columns at 5 steps, us:
+// CG 64^3 two columns 222 / 262, three 259 / 380; 32^3 188 / 206, 206 / 292).  Both
+// take equally long at about 5, 10 and 15 steps for two columns of 12^3 (2 tiles),
+// 32^3 (32) and 64^3 (256), and at 8, 23 and 60 for three.
+inline bool columns_pay(int nrhs, int tiles, const SolveArgs& a) {
+    const int each = tiles <= 2 ? 4 : tiles <= 64 ? 12 : 16;
+    return a.max_steps <= 0 || a.max_steps >= std::max(kResMinSteps, each * (nrhs - 1));
+}
+
 #define GIS_NR_DISPATCH(nrhs, NRC, ...)                     \
     switch (nrhs) {                                         \
         case 1: { constexpr int NRC = 1; __VA_ARGS__; } break; \
@@ -834,7 +844,8 @@ int device_solve_multi(gis_context* h, int method, int nrhs, bool transpose, con
     GIS_TRY(ensure_valT(h));
     int worst = kOK, first = 0;
     // a few columns of a system that fits the chip: one resident solve each
-    if (nrhs <= kResColumns && (method == 0 ? resident_cg_fits(h) : resident_bicg_fits(h))) {
+    if (nrhs <= kResColumns && columns_pay(nrhs, tiles_of(h->N), a) &&
+        (method == 0 ? resident_cg_fits(h) : resident_bicg_fits(h))) {
         GIS_TRY(solve_columns(h, method, nrhs, transpose, a, X, B, iters, norm0, normf, status,
                               &first, &worst));
         if (first == nrhs) return worst;

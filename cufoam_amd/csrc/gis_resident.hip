@@ -982,7 +982,7 @@ int resident_cg(gis_context* h, const Mat<double>& m, double* r, double* p, doub
     *ran = false;
     bool tab;
     const int rpt = res_cg_tiles(h);
-    if (!res_form(h, kResCg, &tab) || rpt == 0) return kOK;
+    if (!res_form(h, kResCg, &tab) || rpt == 0 || iteration_budget(h) < kResMinSteps) return kOK;
     const dim3 g((unsigned)((tiles_of(h->N) + rpt - 1) / rpt));
     return run_resident(h, kResCg, [&](const ResWs& ws) {
         const auto go = [&](auto k) {
@@ -1003,7 +1003,9 @@ int resident_bicg(gis_context* h, const Mat<double>& m, const Mat<double>& mt, d
                   double* rs, double* p, double* ps, double* qx, double* x, bool* ran) {
     *ran = false;
     bool tab;
-    if (!resident_bicg_fits(h) || !res_form(h, kResBicg, &tab)) return kOK;
+    if (!resident_bicg_fits(h) || !res_form(h, kResBicg, &tab) ||
+        iteration_budget(h) < kResMinSteps)
+        return kOK;
     const dim3 g((unsigned)tiles_of(h->N));
     return run_resident(h, kResBicg, [&](const ResWs& ws) {
         const auto go = [&](auto k) {

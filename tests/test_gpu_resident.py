@@ -356,3 +356,32 @@ def test_columns_that_do_not_fit_go_together(gpu):
             ref = O.solve("BiCG", A, B[k], np.zeros(s.n_cells), 0.0, 40, At=At)
             assert it[k] == ref.iterations and nf[k] == ref.hist[-1]
             np.testing.assert_array_equal(X[k], ref.x)
+
+
+@pytest.mark.parametrize("edge", [12, 30, 48])
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+def test_few_steps_run_as_stages(gpu, edge, method):
+    """Solves capped below the steps from which a resident launch pays: the stages,
+    and for several columns one SpMM solve."""
+    s = mesh.laplacian(edge, seed=13, shift=0.1, symmetric=method == "CG")
+    gpu.set_system(s)
+    A = O.ldu2csr(s)
+    for steps, ran in ((1, {}), (2, {}), (3, {"ran": 1})):
+        (x, hist, _), grew = counted(
+            gpu, lambda g: g.solve(method, s.b, s.x0, error=0.0, max_steps=steps))
+        assert grew == ran
+        ref = O.solve(method, A, s.b, s.x0, 0.0, steps)
+        np.testing.assert_array_equal(hist, ref.hist)
+        np.testing.assert_array_equal(x, ref.x)
+    B = np.random.default_rng(5).uniform(-1, 1, (3, s.n_cells))
+    each = {12: 4, 30: 12, 48: 16}[edge]
+    for nrhs in (1, 2, 3):
+        line = max(3, each * (nrhs - 1))
+        for steps, ran in ((line - 1, {}), (line, {"ran": nrhs})):
+            (X, it, nf, _), grew = counted(
+                gpu, lambda g: g.solve_multi(method, B[:nrhs], None, error=0.0, max_steps=steps))
+            assert grew == ran
+            for k in range(nrhs):
+                ref = O.solve(method, A, B[k], np.zeros(s.n_cells), 0.0, steps)
+                assert it[k] == ref.iterations and nf[k] == ref.hist[-1]
+                np.testing.assert_array_equal(X[k], ref.x)
