@@ -683,13 +683,6 @@ __device__ __forceinline__ void tile_sell_c(const int* __restrict__ soff,
     wave_sync_lds();
 }
 
-// Bit j + u of a row mask, for slot u of the batch that starts at slot j: a batch
-// may reach past a table of 32 entries (j <= 31, u < 32), where the bit is 0.
-// Two shifts, each by less than the mask's width.
-constexpr unsigned slot_bit(unsigned mask, int j, int u) { return ((mask >> j) >> u) & 1u; }
-static_assert(slot_bit(~0u, 28, 3) == 1u && slot_bit(~0u, 28, 4) == 0u &&
-              slot_bit(~0u, 28, 6) == 0u, "slots past a table of 32 entries are absent");
-
 // Slices with a column-offset table (SellD): the slice's rows share a sorted
 // list of U column offsets (doffs[ooff[s] ..]); slot k of a row holds column
 // row + doffs[ooff[s] + k] when bit k of the row's mask is set, and is a
@@ -704,10 +697,11 @@ static_assert(slot_bit(~0u, 28, 3) == 1u && slot_bit(~0u, 28, 4) == 0u &&
 // (scalar) offset table, not on the mask: values, masks and gathers of a batch
 // are all in flight together, one memory round trip per batch.
 //
-// B: slots per batch.  FP32 kernels take 7 where no table is longer (the 7-point
-// stencil): with 8 the last slot of every batch is read and gathered a second
-// time (mixed CG at 256^3 191.3 -> 185.4 us per iteration, at 160^3 59.6 -> 58.6; FP64
-// CG unchanged, 366.9).
+// B: slots per batch: 8, whose last batch ends at slot 31 as a table does, or 7 for
+// tables of at most 7 (a later batch of 7 could reach past the mask).  FP32 kernels
+// take 7 where no table is longer (the 7-point stencil): with 8 the last slot of
+// every batch is read and gathered a second time (mixed CG at 256^3 191.3 -> 185.4 us
+// per iteration, at 160^3 59.6 -> 58.6; FP64 CG unchanged, 366.9).
 template <typename T, int B, class XOp>
 __device__ __forceinline__ T sell_row_d(const int* __restrict__ offs, unsigned mask,
                                         const T* __restrict__ dval, int a, int len, int lane,
@@ -727,7 +721,7 @@ __device__ __forceinline__ T sell_row_d(const int* __restrict__ offs, unsigned m
         for (int u = 0; u < B; ++u) xv[u] = xop(min(max(row + o[u], 0), last));
 #pragma unroll
         for (int u = 0; u < B; ++u) {
-            const bool on = slot_bit(mask, j, u);
+            const bool on = (mask >> (j + u)) & 1u;
             const T t = acc + v[u] * xv[u];
             acc = on ? t : acc;
         }
@@ -766,7 +760,7 @@ __device__ __forceinline__ void sell_row2_d(const int* __restrict__ offs0, unsig
         }
 #pragma unroll
         for (int u = 0; u < B; ++u) {
-            const bool on0 = slot_bit(m0, j, u), on1 = slot_bit(m1, j, u);
+            const bool on0 = (m0 >> (j + u)) & 1u, on1 = (m1 >> (j + u)) & 1u;
             const T t0 = acc0 + v0[u] * x0[u];
             const T t1 = acc1 + v1[u] * x1[u];
             acc0 = on0 ? t0 : acc0;
@@ -901,7 +895,7 @@ __device__ __forceinline__ void sell_row2_ds(const int4* __restrict__ tab0, unsi
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const bool on0 = slot_bit(m0, j, u), on1 = slot_bit(m1, j, u);
+            const bool on0 = (m0 >> (j + u)) & 1u, on1 = (m1 >> (j + u)) & 1u;
             const T t0 = acc0 + v0[u] * x0[u];
             const T t1 = acc1 + v1[u] * x1[u];
             acc0 = on0 ? t0 : acc0;
@@ -929,7 +923,7 @@ __device__ __forceinline__ T sell_row_ds(const int4* __restrict__ tab, unsigned 
         for (int u = 0; u < 8; ++u) xv[u] = xop(min(max(row + e[u].x, 0), last));
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const bool on = slot_bit(mask, j, u);
+            const bool on = (mask >> (j + u)) & 1u;
             const T t = acc + v[u] * xv[u];
             acc = on ? t : acc;
         }

@@ -29,6 +29,21 @@ constexpr int kMaxRhs = 8;
 __device__ __forceinline__ double fmat(double a, double b, double c) { return fma(a, b, c); }
 __device__ __forceinline__ float fmat(float a, float b, float c) { return fmaf(a, b, c); }
 
+// Slots of an offset table that sell_multi takes at a time, and whether it takes a
+// batch at slot j of U: not for the last 3 or fewer, which cost less one by one.  A
+// table of 32 counts as one of 31, so that no batch ends past the 32 bits of a row
+// mask (written as another bound on j, the 4-column kernels were 2-6% slower).
+constexpr int kMultiBatch = 7;
+constexpr bool batch_at(int j, int U) { return j == 0 || (U < 31 ? U : 31) - j > 3; }
+
+constexpr bool batches_in_mask() {
+    for (int U = 1; U <= 32; ++U)
+        for (int j = 0; batch_at(j, U); j += kMultiBatch)
+            if (j + kMultiBatch > 32) return false;
+    return true;
+}
+static_assert(batches_in_mask(), "no shift by the mask's width or more");
+
 // y[c][k] for the four 64-row slices of this wave, columns with bit k set in
 // `active`.  A slice with a column-offset table (m.ooff set: the handle's
 // schedule is SellD) reads 64 values per table entry and the row masks; the
@@ -61,10 +76,10 @@ __device__ __forceinline__ void sell_multi(const Mat<T>& m, int N, int row0, XOp
             // a 7-point slice in one batch: every value load and gather of the slice
             // in flight together, none twice (batches of 8 read the last slot
             // again for every column: 3-RHS BiCG at 128^3 234.6 -> 226.9 us per
-            // iteration); up to 3 entries left over are taken one by one
-            constexpr int kB = 7;
+            // iteration); up to 3 entries left over (4 of 32) are taken one by one
+            constexpr int kB = kMultiBatch;
             int j = 0;
-            for (; j == 0 || U - j > 3; j += kB) {
+            for (; batch_at(j, U); j += kB) {
                 T v[kB];
                 int o8[kB], cc[kB];
                 // the offsets as one block of scalar loads before any use: loaded
@@ -78,7 +93,7 @@ __device__ __forceinline__ void sell_multi(const Mat<T>& m, int N, int row0, XOp
                 for (int u = 0; u < kB; ++u) cc[u] = min(max(row + o8[u], 0), last);
 #pragma unroll
                 for (int u = 0; u < kB; ++u) {
-                    const bool on = slot_bit(mask, j, u);
+                    const bool on = (mask >> (j + u)) & 1u;
 #pragma unroll
                     for (int k = 0; k < NR; ++k) {
                         const bool use = on && ((active >> k) & 1u);
