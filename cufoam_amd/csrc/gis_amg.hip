@@ -1087,6 +1087,7 @@ void AmgData::clear() {
     dic_cells_b.release();
     dic_rd.release();
     dic_y.release();
+    sweep_tick.release();
 }
 
 // ---------------------------------------------------------------------------
@@ -1188,7 +1189,34 @@ __global__ __launch_bounds__(kBlk) void k_dic_bwd(int ncell, const int* __restri
 constexpr int kSweepRows = 512;
 constexpr int kSweepThreads = 2 * kSweepRows;
 constexpr int kSweepDeps = 4;    // a row's first dependencies; more are read in turn
-constexpr int kSweepSpins = 1 << 20;
+constexpr int kSweepSpins = 1 << 20;   // polls in vain until a wave looks at the grid's progress
+constexpr int kTickWords = 64, kTickStride = 16;   // progress words, a cache line apart
+
+// A sweep's waits are bounded by the progress of its grid, not by their own
+// length: a workgroup may wait for hundreds before it, each of them milliseconds
+// long where rows have many dependencies.  While a workgroup finishes rows, its
+// watching wave stamps a word; a wave that waited `limit` polls in vain gives up
+// only if no word has changed since it last looked.
+struct SweepWait {
+    unsigned* tick;
+    int limit, fault;   // fault > 0 (gis_set_slot_fault): nothing fetched is ever there
+    unsigned seen = 0;
+    bool looked = false;
+    __device__ SweepWait(unsigned* t, int polls, int f)
+        : tick(t), limit(f > 0 ? f : polls), fault(f) {}
+    __device__ void stamp() const {   // one lane
+        __hip_atomic_store(tick + blockIdx.x % kTickWords * kTickStride, (unsigned)wall_clock64(),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ bool stuck() {   // a whole wave
+        const unsigned now = __hip_atomic_load(tick + (threadIdx.x & 63) * kTickStride,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool still = looked && !__any(now != seen);
+        seen = now;
+        looked = true;
+        return still;
+    }
+};
 
 enum : int { kSweepFactor = 0, kSweepFwd = 1, kSweepBwd = 2 };
 
@@ -1254,6 +1282,40 @@ __device__ __forceinline__ void st_lds(double* p, double v) {
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// A workgroup's watching wave (its first fetching one, once its own values are
+// there), until the compute waves are through: it stamps the progress of their
+// rows, and tells them to give up when the whole grid stands still.  The compute
+// waves, whose turns are the dependency chain, are spared both (there, the look at
+// the stamps made a sweep 1 to 10% longer).
+__device__ __forceinline__ void watch_rows(const double* rows, const int* finished, int* failed,
+                                           SweepWait& wait) {
+    constexpr int kWaves = kSweepRows / 64, kLook = 1024;
+    const int lane = threadIdx.x & 63;
+    int had = 0;
+    for (int polls = 0, waited = 0;;) {
+        if (__hip_atomic_load(finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == kWaves) {
+            if (lane == 0) wait.stamp();
+            return;
+        }
+        if (__hip_atomic_load(failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) return;
+        __builtin_amdgcn_s_sleep(16);   // about 0.4 us: a quarter of a fetching wave's poll
+        if (++polls % kLook == 0) {
+            int have = 0;
+            for (int w = 0; w < kWaves; ++w)
+                have += __popcll(__ballot(!slot_empty_hi(ld_lds(&rows[w * 64 + lane]))));
+            if (have != had && lane == 0) wait.stamp();
+            had = have;
+        }
+        if (++waited / 4 >= wait.limit) {
+            if (wait.stuck()) {
+                __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                return;
+            }
+            waited = 0;
+        }
+    }
+}
+
 // MODE kSweepFactor: out[c] = diag[c] - sum upper lower / out[owner] (a = diag,
 // b = upper, c2 = lower); kSweepFwd: out[c] = rD r[c] - sum rD coef out[owner]
 // (a = r, b = coef); kSweepBwd: out[c] = a[c] - sum rD coef out[neighbour] in
@@ -1264,13 +1326,14 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
     int N, SweepMap map, int base, const int* __restrict__ rowptr, const int* __restrict__ nlow,
     const int* __restrict__ col, const int* __restrict__ perm, const double* __restrict__ rD,
     const double* a, const double* __restrict__ b, const double* __restrict__ c2, double* out,
-    double* clear, KState* st) {
+    double* clear, KState* st, unsigned* tick, int polls) {
     if (st->done) return;
+    SweepWait wait(tick, polls, st->slot_fault);
     constexpr int D = kSweepDeps;
     // this workgroup's rows, then the fetched values per dependency and row,
     // and a 1 that rows with fewer dependencies read
     __shared__ double zz[(1 + D) * kSweepRows + 1];
-    __shared__ int failed;
+    __shared__ int failed, finished;   // finished: compute waves whose rows are done
     const double empty = __longlong_as_double(static_cast<long long>(kSlotEmpty));
     const int tid = threadIdx.x;
     const bool fetch = tid >= kSweepRows;
@@ -1280,7 +1343,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
     const int row = own.row(li, N);
     const bool in = row < N;
     if (tid == 0) {
-        failed = 0;
+        failed = finished = 0;
         st_lds(&zz[(1 + D) * kSweepRows], 1.0);
     }
     if (!fetch) st_lds(&zz[li], empty);
@@ -1343,7 +1406,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
                 if ((pending >> k) & 1u) v[k] = ld_agent(out + at[k]);
 #pragma unroll
             for (int k = 0; k < D; ++k)
-                if (((pending >> k) & 1u) && !slot_empty(v[k])) {
+                if (((pending >> k) & 1u) && !slot_empty(v[k]) && wait.fault <= 0) {
                     st_lds(&zz[(1 + k) * kSweepRows + li], v[k]);
                     pending &= ~(1u << k);
                 }
@@ -1351,12 +1414,17 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
                 spins = 0;
                 continue;
             }
-            if (++spins >= kSweepSpins) {
-                __hip_atomic_store(&failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                break;
+            if (++spins >= wait.limit) {
+                if (wait.stuck()) {
+                    __hip_atomic_store(&failed, 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                    break;
+                }
+                spins = 0;
             }
             __builtin_amdgcn_s_sleep(1);
         }
+        if (tid == kSweepRows + (tid & 63)) watch_rows(zz, &finished, &failed, wait);
         return;
     }
     // Every turn reads all D values and forms the row's from them: rows whose
@@ -1365,7 +1433,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
     bool done = !in, applied = nd <= D;
     bool first_done = false;   // a longer row: its first D are in w
     int kx = n1;               // its next dependency
-    for (int idle = 0;;) {
+    for (;;) {
         double z[D];
 #pragma unroll
         for (int k = 0; k < D; ++k) z[k] = ld_lds(&zz[at[k]]);
@@ -1403,14 +1471,14 @@ __global__ __launch_bounds__(kSweepThreads) void k_ilu_sweep(
                 }
             }
         }
-        if (__all(done)) return;
-        if (__any(moved)) {
-            idle = 0;
-            continue;
+        if (__all(done)) {
+            if ((tid & 63) == 0)
+                __hip_atomic_fetch_add(&finished, 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+            return;
         }
-        if (++idle >= 16 * kSweepSpins ||
-            __hip_atomic_load(&failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
-            break;
+        if (__any(moved)) continue;
+        if (__hip_atomic_load(&failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
         __builtin_amdgcn_s_sleep(1);
     }
     if ((tid & 63) == 0) slot_fail(st, 1);
@@ -1561,6 +1629,10 @@ SweepMap sweep_map(const gis_context* h) {
                     (ny + kBrick - 1) / kBrick};
 }
 
+inline int sweep_polls(const gis_context* h) {
+    return h->sweep_polls > 0 ? h->sweep_polls : kSweepSpins;
+}
+
 inline dim3 sweep_grid(const gis_context* h) { return dim3((unsigned)h->amg->sweep_blocks); }
 
 // kind 4: DIC (the factor from upper alone), 5: DILU (upper and lower)
@@ -1574,7 +1646,10 @@ int ilu_prepare(gis_context* h, int kind) {
     }
     AmgData& A = *h->amg;
     const bool planned = h->upper_tri ? A.sweep_ready : A.dic_levels;
-    if (h->upper_tri) GIS_HIP(h, A.dic_y.ensure(sizeof(double) * (size_t)h->N));
+    if (h->upper_tri) {
+        GIS_HIP(h, A.dic_y.ensure(sizeof(double) * (size_t)h->N));
+        GIS_HIP(h, A.sweep_tick.ensure(sizeof(unsigned) * kTickWords * kTickStride));
+    }
     if (!planned) {
         int st = kOK;
         try {
@@ -1601,7 +1676,7 @@ int ilu_prepare(gis_context* h, int kind) {
                                h->stream, N, sweep_map(h), 0, h->rowptr.as<int>(), h->nbr_cnt.as<int>(),
                                h->col.as<int>(), h->perm.as<int>(), nullptr,
                                h->diag.as<double>(), h->upper.as<double>(), lower, F, nullptr,
-                               h->st);
+                               h->st, A.sweep_tick.as<unsigned>(), sweep_polls(h));
             GIS_HIP(h, hipGetLastError());
             GIS_TRY(read_state(h));
             if (h->st_host->status == kErrSync)
@@ -1644,11 +1719,11 @@ int ilu_apply(gis_context* h, const double* r, double* z, const double* cf, cons
         hipLaunchKernelGGL(k_ilu_sweep<kSweepFwd>, sweep_grid(h), dim3(kSweepThreads), 0,
                            h->stream, N, sweep_map(h), 0, h->rowptr.as<int>(), h->nbr_cnt.as<int>(),
                            h->col.as<int>(), h->perm.as<int>(), A.dic_rd.as<double>(), r, cf,
-                           nullptr, y, z, h->st);
+                           nullptr, y, z, h->st, A.sweep_tick.as<unsigned>(), sweep_polls(h));
         hipLaunchKernelGGL(k_ilu_sweep<kSweepBwd>, sweep_grid(h), dim3(kSweepThreads), 0,
                            h->stream, N, sweep_map(h), h->M + N, h->rowptr.as<int>(), h->nbr_cnt.as<int>(),
                            h->col.as<int>(), h->perm.as<int>(), A.dic_rd.as<double>(), y, cb,
-                           nullptr, z, y, h->st);
+                           nullptr, z, y, h->st, A.sweep_tick.as<unsigned>(), sweep_polls(h));
         GIS_HIP(h, hipGetLastError());
         return kOK;
     }

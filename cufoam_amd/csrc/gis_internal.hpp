@@ -158,6 +158,7 @@ struct AmgData {
     // single-launch sweeps: the bricks' order and the box's strides (0: consecutive rows)
     bool sweep_ready = false;
     DevMem sweep_order;
+    DevMem sweep_tick;            // where the workgroups of a sweep stamp their progress
     int sweep_sx = 0, sweep_sy = 0, sweep_blocks = 0;
     void clear();
     ~AmgData();
@@ -246,6 +247,7 @@ struct gis_context {
     long long res_count[gis::kResCounts] = {};  // gis_get_resident_counts
     int res_skip = 0, res_backoff = 0;          // solves held back after a late grid
     int late_after = 0, late_n = 0;             // gis_set_late_launches (failure-path tests)
+    int sweep_polls = 0;                        // gis_set_sweep_polls (the same); 0: the default
 
     gis::Schedule sched;
     gis::Timer timer;

@@ -359,13 +359,17 @@ GIS_API int gis_set_gamg(gis_handle h, double omega, int nu, double cscale);
  * polls > 0 every workgroup that collects reduction partials on the device
  * treats them as never written and gives up after `polls` polls, so every
  * solve (and dot / NormFactor) of the handle on more than one 1024-row tile
- * stops with GIS_ERR_SYNC; polls = 0 restores normal operation.  The kernels
+ * stops with GIS_ERR_SYNC, and so does a DIC / DILU sweep on more than one block of
+ * 512 rows; polls = 0 restores normal operation.  The kernels
  * still exit normally.  Applies to solves started after the call. ---- */
 GIS_API int gis_set_slot_fault(gis_handle h, int polls);
 /* Failure-path tests only: after `after` more resident launches of the handle,
  * `count` of them find their workgroups not all there in time and give up (the
  * kernels exit normally); a launch of one workgroup waits for nobody. */
 GIS_API int gis_set_late_launches(gis_handle h, int after, int count);
+/* Failure-path tests only: polls in vain after which a waiting wave of a DIC / DILU
+ * sweep looks whether the sweep gets on at all (0: the default, 2^20). */
+GIS_API int gis_set_sweep_polls(gis_handle h, int polls);
 /* The hierarchy (built if needed): level count, then one level's sizes,
  * aggregation map (cell -> next-level cell; levels below the last) and LDU
  * matrix (any output pointer may be NULL). */

@@ -102,3 +102,57 @@ def test_addressing_not_upper_triangular(gpu):
     x, hist, st = gpu.solve_pcg("DIC", s.b, s.x0, error=0.0, max_steps=4)
     np.testing.assert_array_equal(hist, ref.hist)
     np.testing.assert_array_equal(x, ref.x)
+
+
+@pytest.mark.parametrize("kind", ["DIC", "DILU"])
+def test_long_chains_are_waited_for(gpu, kind):
+    """40 workgroups in a chain, each slow (24 dependencies a row, most of them read
+    one by one): a wave waits many times the polls after which it looks at the
+    grid's progress, and gives up only if there is none."""
+    n, bands = 40 * 512, 24
+    c = np.arange(n)
+    la = np.concatenate([c[:n - d] for d in range(1, bands + 1)])
+    ua = np.concatenate([c[d:] for d in range(1, bands + 1)])
+    s = build(n, la, ua, 11, kind == "DIC")
+    gpu.set_system(s)
+    gpu.set_sweep_polls(1 << 15)
+    try:
+        if kind == "DIC":
+            ref = O.pcg("DIC", s, s.b, s.x0, 0.0, 2)
+            x, hist, st = gpu.solve_pcg("DIC", s.b, s.x0, error=0.0, max_steps=2)
+        else:
+            ref = O.pbicg_ldu("DILU", s, s.b, s.x0, 0.0, 2)
+            x, hist, st = gpu.solve_pbicg("DILU", s.b, s.x0, error=0.0, max_steps=2)
+    finally:
+        gpu.set_sweep_polls(0)
+    np.testing.assert_array_equal(hist, ref.hist)
+    np.testing.assert_array_equal(x, ref.x)
+
+
+@pytest.mark.parametrize("kind", ["DIC", "DILU"])
+def test_sweep_failure_is_reported_and_recovers(gpu, kind):
+    """The sweeps' bounded wait, forced from the host (gis_set_slot_fault): 1000
+    rows are one reduction tile, which waits for nobody, but two workgroups of a
+    sweep.  The factor's sweep and, with the factor kept, the solve's give up with
+    GIS_ERR_SYNC; then the refilled vectors give the same bits again."""
+    from cufoam_amd.gis import GisError
+    s = dense_rows(1000, 12, kind == "DIC")
+    ref = (O.pcg("DIC", s, s.b, s.x0, 0.0, 5) if kind == "DIC"
+           else O.pbicg_ldu("DILU", s, s.b, s.x0, 0.0, 5))
+
+    def solve():
+        call = gpu.solve_pcg if kind == "DIC" else gpu.solve_pbicg
+        return call(kind, s.b, s.x0, error=0.0, max_steps=5)
+    gpu.set_system(s)
+    for kept in (False, True):   # whether the factor is there already
+        gpu.set_slot_fault(4)
+        try:
+            with pytest.raises(GisError) as e:
+                solve()
+            assert e.value.status == 13
+        finally:
+            gpu.set_slot_fault(0)
+        for _ in range(2):
+            x, hist, st = solve()
+            np.testing.assert_array_equal(hist, ref.hist)
+            np.testing.assert_array_equal(x, ref.x)
