@@ -160,12 +160,12 @@ __device__ __forceinline__ int xcd_tile(int i, int G) {
     return x * q + min(x, r) + j;
 }
 
-// Workgroup i's tile when each XCD takes c consecutive tiles at a time (c <= 0: one,
-// the dispatch order).  Tiles 8 c apart then share an XCD, whose L2 holds what a
+// Workgroup i's tile (group of tiles) when each XCD takes c consecutive ones at a time
+// (c <= 0: one, the dispatch order).  Tiles 8 c apart then share an XCD, whose L2 holds what a
 // row's far neighbours need: c is an eighth of the farthest offset's distance in
 // tiles where that is no multiple of 8 (mat_chunk).  Past the last whole span of 8 c
 // tiles the dispatch order goes on.  A group's last tile may go out up to 8 c
-// workgroups early; its collector waits for those few.
+// workgroups early; its collector waits for those.
 __device__ __forceinline__ int chunk_tile(int i, int T, int c) {
     if (c <= 0) return i;
     const int span = kXcds * c;
@@ -202,6 +202,8 @@ struct SuperTile {
         tile0 = s * C;
         nt = min(C, tiles_of(N) - tile0);
     }
+    // chunk in workgroups, C tiles each (divided by C the mixed passes were 1%
+    // slower at 160^3 and 200^3 with C = 2, the others equal)
     __device__ SuperTile(int N, int chunk) {
         tile0 = chunk_tile((int)blockIdx.x, (int)gridDim.x, chunk) * C;
         nt = min(C, tiles_of(N) - tile0);
@@ -366,12 +368,21 @@ inline dim3 super_grid(int N, int C) { return dim3((unsigned)((tiles_of(N) + C -
 // of 8 already.  Per iteration, without / with (FP64 CG and mixed): 160^3 99.4 /
 // 91.3 and 57.8 / 56.0 us, 200^3 189.3 / 184.9 and 103.1 / 97.6, 245^3 351.1 / 348.4
 // and 184.3 / 172.3; not below (140^3, P 19: 71.8 / 71.7 and 44.3 / 44.7) nor at
-// 256^3 (P 64: 376.5 / 377.3 and 192.9 / 194.2).
+// 256^3 (P 64: 376.5 / 377.3 and 192.9 / 194.2).  Only where the offset is a plane of
+// at least four: a pair of cyclic patches, whose offset is nearly the whole mesh, would
+// give each XCD an eighth of it and its collectors as long to wait (160^3 with such a
+// pair, with / without: CG 111.2 / 109.2 us, mixed 68.2 / 69.4).
+constexpr int chunk_of(long long offset, long long tiles) {
+    constexpr long long kSpan = kXcds * kTile;
+    const long long c = (offset + kSpan / 2) / kSpan;
+    return c >= 3 && offset % kSpan != 0 && tiles >= 4 * kXcds * c ? (int)c : 0;
+}
+static_assert(chunk_of(160 * 160, 4000) == 3 && chunk_of(245 * 245, 14362) == 7, "box planes");
+static_assert(chunk_of(256 * 256, 16384) == 0, "a multiple of 8 tiles");
+static_assert(chunk_of(159 * 160 * 160, 4000) == 0, "the halves of a cyclic pair");
+
 inline int mat_chunk(const gis_context* h) {
-    constexpr int kSpan = kXcds * kTile;
-    const int off = h->lay_max_offset;
-    const int c = (off + kSpan / 2) / kSpan;
-    return c >= 3 && off % kSpan != 0 ? c : 0;
+    return chunk_of(h->lay_max_offset, tiles_of(h->N));
 }
 
 inline Mat<double> mat64(const gis_context* h) {
