@@ -1571,6 +1571,16 @@ __global__ __launch_bounds__(kBlk) void k_box_check(int N, int sx, int sy,
     if (__any(wrong) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
+// Whether bx x by x bz bricks serve a box of N cells.  Flat boxes would leave most of
+// a brick's threads without a cell; and the places of a brick that sticks out,
+// which SweepBlock::row forms before it drops them, must be ints.
+constexpr bool bricks_pay(long long bx, long long by, long long bz, long long N) {
+    const long long places = bx * by * bz * kSweepRows;
+    return places <= 4 * N + kSweepRows && places <= INT_MAX;
+}
+static_assert(bricks_pay(8, 8, 8, 64 * 64 * 64) && !bricks_pay(8, 7, 1, 60 * 50), "");
+static_assert(!bricks_pay(2165, 2165, 1, 2LL * 17320 * 17320), "rows past the int range");
+
 // The pattern's sweep map: bricks where it is a box of cells, else consecutive
 // rows.
 int sweep_plan(gis_context* h) {
@@ -1597,8 +1607,7 @@ int sweep_plan(gis_context* h) {
     const int nx = sx, ny = sy / sx, nz = (h->N + sy - 1) / sy;
     const int bx = (nx + kBrick - 1) / kBrick, by = (ny + kBrick - 1) / kBrick,
               bz = (nz + kBrick - 1) / kBrick;
-    // flat boxes would leave most of a brick's threads without a cell
-    if ((long long)bx * by * bz * kSweepRows > 4LL * h->N + kSweepRows) return kOK;
+    if (!bricks_pay(bx, by, bz, h->N)) return kOK;
     int bad = 1;
     GIS_HIP(h, hipMemsetAsync(d + 2, 0, sizeof(int), h->stream));
     hipLaunchKernelGGL(k_box_check, grid_of(h->N), dim3(kBlk), 0, h->stream, h->N, sx, sy,
