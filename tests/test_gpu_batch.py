@@ -41,10 +41,16 @@ def test_batch_bit_exact_vs_oracle(gpu, use_graph, schedule, direction):
             off += s.n_cells
 
 
-def test_batch_graph_replays_with_interleaved_work(gpu):
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_graph_replays_with_interleaved_work(gpu, graph):
+    """graph: the schedule is chosen explicitly, which switches resident launches off,
+    so that the stages' graph is captured and replayed."""
     import torch
     systems = _systems([6, 11, 4], 20)
     gpu.batch_set_systems(systems)
+    if graph:
+        gpu.set_schedule(spmv64=gpu.get_schedule()["spmv64"])
+    before = gpu.resident_counts()["ran"]
     b = np.concatenate([s.b for s in systems])
     err = np.full(3, 1e-10)
     x0, it0, nf0, _ = gpu.batch_solve(b, None, err, 2000, use_graph=False)
@@ -54,19 +60,25 @@ def test_batch_graph_replays_with_interleaved_work(gpu):
         x, it, nf, _ = gpu.batch_solve(b, None, err, 2000, use_graph=True)
         assert np.array_equal(it, it0) and np.array_equal(nf, nf0)
         np.testing.assert_array_equal(x, x0)
+    assert gpu.resident_counts()["ran"] - before == (0 if graph else 5)
 
 
-def test_batch_64_uneven_systems_equal_single_solves(gpu):
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_64_uneven_systems_equal_single_solves(gpu, graph):
     from cufoam_amd.gis import Gis
     edges = mesh.batch_edges(64, 16, 64, seed=0)
     systems = _systems(edges, 100)
     N = sum(s.n_cells for s in systems)
     print(f"[case] 64 systems, {N} cells in total", flush=True)
     gpu.batch_set_systems(systems)
+    if graph:
+        gpu.set_schedule(spmv64=gpu.get_schedule()["spmv64"])
+    before = gpu.resident_counts()["ran"]
     b = np.concatenate([s.b for s in systems])
     err = np.array([1e-8 * np.linalg.norm(s.b) for s in systems])
     x, it, nf, st = gpu.batch_solve(b, None, err, 5000, use_graph=True)
     assert np.all(st == 0)
+    assert (gpu.resident_counts()["ran"] > before) == (not graph)
     with Gis(0) as single:
         off = 0
         for k, s in enumerate(systems):

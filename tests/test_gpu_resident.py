@@ -72,8 +72,10 @@ def test_resident_equals_stages(gpu, n, method):
 
     def run(g):
         return g.solve(method, s.b, s.x0, error=1e-9, max_steps=40)
-    x, hist, st = run(gpu)
-    x1, hist1, st1 = stages(gpu, run)
+    (x, hist, st), grew = counted(gpu, run)
+    assert grew == ({"ran": 1} if n <= (512 if method == "CG" else 256) * 1024 else {})
+    (x1, hist1, st1), grew = counted(gpu, lambda g: stages(g, run))
+    assert grew == {}
     assert st == st1
     np.testing.assert_array_equal(hist, hist1)
     np.testing.assert_array_equal(x, x1)
@@ -92,7 +94,8 @@ def test_scattered_halos_and_long_rows(gpu, n_cells, n_faces, method):
 
     def run(g):
         return g.solve(method, s.b, s.x0, error=1e-9, max_steps=25)
-    x, hist, _ = run(gpu)
+    (x, hist, _), grew = counted(gpu, run)
+    assert grew == {}
     x1, hist1, _ = stages(gpu, run)
     np.testing.assert_array_equal(hist, hist1)
     np.testing.assert_array_equal(x, x1)
@@ -109,20 +112,40 @@ def test_random_numbering(gpu, n, method):
 
     def run(g):
         return g.solve(method, s.b, s.x0, error=1e-6, max_steps=60)
-    for _ in range(2):
-        x, hist, _ = run(gpu)
+    # 12^3: halos within 2 workgroups; 40^3: about 6000 rows, within CG's 8192, past
+    # BiCG's 4096; 70^3: past CG's 5120 with two tiles, and more tiles than BiCG takes
+    fits = n == 12 or (n == 40 and method == "CG")
+    tries = {"ran": 1} if fits else {} if n == 70 and method == "BiCG" else {"unfit": 1}
+    for want in (tries, tries if fits else {}):
+        (x, hist, _), grew = counted(gpu, run)
+        assert grew == want
     x1, hist1, _ = stages(gpu, run)
     np.testing.assert_array_equal(hist, hist1)
     np.testing.assert_array_equal(x, x1)
 
 
-@pytest.mark.parametrize("n", [5, 14])
+def line(n, shift, sym):
+    """n cells on a line: CG and BiCG take thousands of iterations."""
+    rng = np.random.default_rng(n)
+    la = np.arange(n - 1, dtype=np.int32)
+    up = -(1.0 + 0.5 * rng.random(n - 1))
+    lo = up.copy() if sym else up * (1.0 + 1e-3 * rng.random(n - 1))
+    diag = mesh.row_abs_sum(n, la, la + 1, lo, up) + shift
+    return mesh.LduSystem(n, la, la + 1, diag, lo, up, rng.uniform(-1, 1, n), np.zeros(n))
+
+
+@pytest.mark.parametrize("n", [5, 14, -900, -1900])
 @pytest.mark.parametrize("method", ["CG", "BiCG"])
 def test_chunks_continue(gpu, n, method):
-    """More iterations than one launch makes: the next one goes on where it stopped."""
-    s = mesh.laplacian(n, seed=9, shift=1e-3, symmetric=method == "CG")
+    """More iterations than one launch makes: the next one goes on where it stopped.
+    A box of 5^3 ends within one; 14^3 are three workgroups, lines of 900 and 1900
+    cells a single one of one and of two tiles (BiCG: two workgroups)."""
+    s = (mesh.laplacian(n, seed=9, shift=1e-3, symmetric=method == "CG") if n > 0
+         else line(-n, 1e-6, method == "CG"))
     gpu.set_system(s)
-    x, hist, _ = gpu.solve(method, s.b, s.x0, error=-1.0, max_steps=4100)
+    (x, hist, _), grew = counted(
+        gpu, lambda g: g.solve(method, s.b, s.x0, error=-1.0, max_steps=4100))
+    assert grew == {"ran": -(-(len(hist) - 1) // 2048)} and (grew["ran"] > 1 or n == 5)
     ref = O.solve(method, O.ldu2csr(s), s.b, s.x0, -1.0, 4100)
     np.testing.assert_array_equal(hist, ref.hist)
     np.testing.assert_array_equal(x, ref.x)
@@ -134,7 +157,9 @@ def test_columns_and_transpose(gpu):
     gpu.set_system(s)
     B = np.random.default_rng(2).uniform(-1, 1, (3, s.n_cells))
     for transpose in (False, True):
-        a = gpu.solve_multi("BiCG", B, None, error=1e-8, max_steps=300, transpose=transpose)
+        a, grew = counted(gpu, lambda g: g.solve_multi("BiCG", B, None, error=1e-8,
+                                                       max_steps=300, transpose=transpose))
+        assert grew == {"ran": 3}
         b = stages(gpu, lambda g: g.solve_multi("BiCG", B, None, error=1e-8, max_steps=300,
                                                 transpose=transpose))
         gpu.set_system(s)
@@ -156,16 +181,18 @@ def test_infinite_and_nan_inputs(gpu):
 
             def run(g):
                 return g.solve(method, b, s.x0, error=1e-9, max_steps=6)
-            x, hist, st = run(gpu)
+            (x, hist, st), grew = counted(gpu, run)
+            assert grew == {"ran": 1}
             x1, hist1, st1 = stages(gpu, run)
             assert st == st1
             np.testing.assert_array_equal(hist, hist1)
             np.testing.assert_array_equal(x, x1)
 
 
-@pytest.mark.parametrize("edges", [[1, 2, 10, 11, 13], [40, 64, 3, 65, 17, 30, 30, 30],
-                                   [20] * 40 + [8] * 30])
-def test_batch(gpu, edges):
+@pytest.mark.parametrize("edges,launches", [([1, 2, 10, 11, 13], 1),
+                                            ([40, 64, 3, 65, 17, 30, 30, 30], 2),
+                                            ([20] * 40 + [8] * 30, 1)])
+def test_batch(gpu, edges, launches):
     """One launch, several launches with systems of one and of two tiles per
     workgroup, and many small systems: every system its own solve's bits."""
     systems = [mesh.laplacian(n, seed=50 + i, shift=1e-3) for i, n in enumerate(edges)]
@@ -176,7 +203,8 @@ def test_batch(gpu, edges):
         return g.batch_solve(b, None, err, 70)
     gpu.batch_set_systems(systems)
     for _ in range(2):
-        x, it, nf, st = run(gpu)
+        (x, it, nf, st), grew = counted(gpu, run)
+        assert grew == {"ran": launches}
     gpu.batch_set_systems(systems)
     x1, it1, nf1, st1 = stages(gpu, run)
     np.testing.assert_array_equal(it, it1)
@@ -204,7 +232,8 @@ def test_batch_mixed_fit(gpu):
     mixed = small + [mesh.random_ldu(900, 9000, seed=1, symmetric=True)]
     b = np.concatenate([s.b for s in mixed])
     gpu.batch_set_systems(mixed)
-    x, it, nf, st = gpu.batch_solve(b, None, 1e-8, 300)
+    (x, it, nf, st), grew = counted(gpu, lambda g: g.batch_solve(b, None, 1e-8, 300))
+    assert grew == {}
     off = 0
     for i, s in enumerate(mixed):
         ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, 1e-8, 300)

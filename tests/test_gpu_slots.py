@@ -110,16 +110,26 @@ def test_multi_rhs_global_level2_path():
             assert torch.equal(X[k], x1), k
 
 
-def test_sync_failure_is_reported_and_recovers(gpu):
+@pytest.mark.parametrize("route", ["resident", "stages"])
+def test_sync_failure_is_reported_and_recovers(gpu, route):
     """The collectors' bounded wait, forced from the host (gis_set_slot_fault:
     every collector sees its slots unwritten and gives up after 4 polls; the
     kernels still exit normally): dot, NormFactor, single, mixed, multi-RHS and
     batched solves stop with GIS_ERR_SYNC, and after the hook is cleared the refilled slots give
-    bit-exact results again."""
+    bit-exact results again.  CG, the columns and the batch both as resident launches
+    and, with the schedule chosen explicitly, as one launch per stage and SpMM."""
     from cufoam_amd.gis import GisError
+
+    def on_route():
+        if route == "stages":
+            gpu.set_schedule(spmv64=gpu.get_schedule()["spmv64"])
+
+    steps = 20   # of the columns: enough for resident ones
     s = mesh.laplacian(48, seed=26, shift=1e-2)   # 110,592 rows: 108 tiles, 2 groups
     A = O.ldu2csr(s)
     gpu.set_system(s)
+    on_route()
+    before = gpu.resident_counts()
     B = np.random.default_rng(27).uniform(-1, 1, (2, s.n_cells))
     small = [mesh.laplacian(12, seed=28, shift=1e-3), mesh.laplacian(3, seed=29, shift=1e-3)]
     import torch
@@ -129,11 +139,12 @@ def test_sync_failure_is_reported_and_recovers(gpu):
         for call in (lambda: gpu.dot(b_d, b_d), lambda: gpu.norm_factor(b_d, b_d),
                      lambda: gpu.solve("CG", s.b, s.x0, error=0.0, max_steps=5),
                      lambda: gpu.solve_mixed(s.b, s.x0, 1e-10, 1e-2, 5, 0),
-                     lambda: gpu.solve_multi("BiCG", B, None, error=0.0, max_steps=5)):
+                     lambda: gpu.solve_multi("BiCG", B, None, error=0.0, max_steps=steps)):
             with pytest.raises(GisError) as e:
                 call()
             assert e.value.status == 13
         gpu.batch_set_systems(small)
+        on_route()
         bb = np.concatenate([t.b for t in small])
         with pytest.raises(GisError) as e:   # the 2-tile system fails, the 1-tile one cannot
             gpu.batch_solve(bb, None, 1e-9, 500, use_graph=True)
@@ -148,6 +159,7 @@ def test_sync_failure_is_reported_and_recovers(gpu):
         np.testing.assert_array_equal(x[off:off + t.n_cells], ref.x)
         off += t.n_cells
     gpu.set_system(s)
+    on_route()
     assert gpu.dot(b_d, b_d) == O.dot(s.b, s.b)
     assert gpu.norm_factor(b_d, b_d) == O.norm_factor(A, s.b, s.b)
     ref = O.solve("CG", A, s.b, s.x0, 0.0, 5)
@@ -158,9 +170,13 @@ def test_sync_failure_is_reported_and_recovers(gpu):
     x, hist, it, rel, st = gpu.solve_mixed(s.b, s.x0, 1e-10, 1e-2, 5, 0)
     assert (st, it) == (rst, rit)
     np.testing.assert_array_equal(x, rx)
-    X, its, nfs, sts = gpu.solve_multi("BiCG", B, None, error=0.0, max_steps=5)
+    X, its, nfs, sts = gpu.solve_multi("BiCG", B, None, error=0.0, max_steps=steps)
     At = O.transpose(A)
     for k in range(2):
-        r1 = O.solve("BiCG", A, B[k], np.zeros(s.n_cells), 0.0, 5, At=At)
+        r1 = O.solve("BiCG", A, B[k], np.zeros(s.n_cells), 0.0, steps, At=At)
         assert nfs[k] == r1.hist[-1]
         np.testing.assert_array_equal(X[k], r1.x)
+    grew = {k: v - before[k] for k, v in gpu.resident_counts().items() if v != before[k]}
+    # resident: CG, the columns and the batch, failing (the set-up's reduction fails
+    # first, and the launch ends at once) and recovered
+    assert (set(grew) == {"ran"} and grew["ran"] >= 6) if route == "resident" else not grew
