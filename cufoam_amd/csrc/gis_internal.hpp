@@ -359,8 +359,8 @@ constexpr int kMethodPcg0 = 8;
 constexpr int kMethodPbicgDiag = 13;
 constexpr int kMethodPbicgDilu = 14;
 // DIC / DILU (gis_amg.hip): the reciprocal factored diagonal for kind 4 (DIC)
-// or 5 (DILU), and z = M^-1 r by the level-scheduled sweeps with the forward
-// sweep's coefficients cf and the backward sweep's cb
+// or 5 (DILU), and z = M^-1 r by the sweeps (one launch each, or level by level)
+// with the forward sweep's coefficients cf and the backward sweep's cb
 int ilu_prepare(gis_context* h, int kind);
 int ilu_begin(gis_context* h);   // before a solve's first application
 int ilu_apply(gis_context* h, const double* r, double* z, const double* cf, const double* cb);

@@ -770,7 +770,7 @@ int solve_pbicg_diag(gis_context* h, const SolveArgs& a, double* x, const double
 }
 
 // BiCG preconditioned by OpenFOAM's DILU (no counterpart in the reference):
-// z = M^-1 r and zs = M^-T rs by the level-scheduled sweeps of gis_amg.hip (the
+// z = M^-1 r and zs = M^-T rs by the sweeps of gis_amg.hip (the
 // forward sweep reads lower, the backward one upper; M^-T exchanges them).
 int solve_pbicg_dilu(gis_context* h, const SolveArgs& a, double* x, const double* b) {
     GIS_TRY(ensure_valT(h));

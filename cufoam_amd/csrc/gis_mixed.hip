@@ -256,9 +256,10 @@ __global__ __launch_bounds__(kWG) void k_mx1s(Mat<float> m, int N, const float* 
     tr.end(red, st, shr, [&](const double (&v)[1]) { finish_alpha(st, v[0]); });
 }
 
-// Rows from which k_mx2's tiles are XCD-contiguous; below, k_mx1's order, in which
-// the vectors still cached are met first (mixed CG per iteration, XCD-contiguous /
-// k_mx1's order: 160^3 58.7 / 57.9 us, 180^3 77.0 / 76.5, 200^3 102.8 / 102.8, 224^3
+// Rows from which k_mx2's tiles are XCD-contiguous; below, the dispatch order, k_mx1's
+// where that takes no chunks (mat_chunk), in which the vectors still cached are met
+// first (mixed CG per iteration, XCD-contiguous / dispatch order, before k_mx1 took
+// chunks: 160^3 58.7 / 57.9 us, 180^3 77.0 / 76.5, 200^3 102.8 / 102.8, 224^3
 // 134.9 / 136.3, 256^3 182.6 / 185.0).
 constexpr int kMx2Stream = 1 << 23;
 

@@ -175,9 +175,11 @@ __global__ __launch_bounds__(kWG) void k_cg_dir(int N, const double* __restrict_
                                                 double* __restrict__ pb1,
                                                 double* __restrict__ x, const KState* st) {
     if (st->done) return;
-    // the SpMV's tile order: what its neighbours in the iteration read or wrote is
-    // then met in the same order (256^3: 375.9 -> 366.9 us per iteration against
-    // XCD-contiguous tiles, k_cg2 likewise at 128^3: 54.2 -> 52.7)
+    // the dispatch order, the SpMV's where it takes no chunks (mat_chunk): what its
+    // neighbours in the iteration read or wrote is then met in the same order
+    // (against XCD-contiguous tiles here and in k_cg2, per iteration 256^3 375.9 ->
+    // 366.9 us, 128^3 54.2 -> 52.7; a whole 128^3 solve with its copies 45.7 -> 44.9 ms,
+    // where two runs of one side differ by 0.6)
     const SuperTile<C> sup(N, false);
     const int k = st->k + 1;
     const double* p_old = (k & 1) ? pb0 : pb1;

@@ -180,14 +180,19 @@ typedef struct gis_schedule {
  * timing: the autotuner's cached choice for (device, N, nnz) if there is one,
  * else schedule 6 (FP64 direction form 1, FP32 form 0) when the slices
  * with a column-offset table hold at least 95% of the sliced-row slots
- * (structured meshes, batches of them), else schedule 0. */
+ * (structured meshes, batches of them), else schedule 0.
+ * A schedule describes the launch-per-stage kernels: choosing an FP64 field here
+ * (spmv64, fp64_direction or coarsen64, also to the value in force) switches
+ * resident solves off (gis_resident_counts) until the next pattern, which makes
+ * small systems up to 2.8 times slower. */
 GIS_API int gis_set_schedule(gis_handle h, const gis_schedule *s);
 GIS_API int gis_get_schedule(gis_handle h, gis_schedule *s);
 
 /* ---- resident solves (no counterpart in the reference): CG, BiCG and batched CG
  * of systems that fit the chip run as one launch per solve, or per 2048 iterations,
- * whose workgroups start together or not at all; otherwise the solve runs one
- * launch per stage.  Counts since gis_create. ---- */
+ * whose workgroups start together or not at all; otherwise, and for solves capped
+ * at one or two steps, the solve runs one launch per stage.  Same bits either way.
+ * Counts since gis_create. ---- */
 typedef struct {
     long long ran;      /* launches that ran */
     long long unfit;    /* launches that gave up: too many rows of other workgroups are
@@ -223,7 +228,8 @@ GIS_API int gis_autotune_clear(void);
  * iteration, 1 = the vector-update kernel of each iteration, 2 = the FP64
  * update kernel of gis_solve_mixed, 3 = gis_spmv*_device_async, 4 = the
  * separate CG direction pass (direction form 1).  Each timed
- * launch adds two event records to the stream. ---- */
+ * launch adds two event records to the stream.  Slots 0, 1 and 4 time the launches
+ * of the stages: while one of them is recorded, no resident solve runs. ---- */
 GIS_API int gis_set_timing(gis_handle h, int slot_mask);
 GIS_API int gis_get_timing(gis_handle h, int slot, double *total_ms, long long *count);
 /* Time one launch in `period` (>= 1, default 1) of each recorded slot: each
@@ -309,15 +315,16 @@ GIS_API int gis_set_coupled_values_device(gis_handle h, const double *d_diag,
 /* OpenFOAM's DIC (diagonal incomplete Cholesky) from its published algorithm:
  * rD = 1 / (diag - sum over lower faces of upper^2 rD_owner) in face order,
  * z = rD r, a forward sweep over the faces and a backward sweep in reverse face
- * order.  The sweeps run level by level (cells whose faces are independent),
- * one launch per level: about 3n launches per application on an n^3 mesh.
+ * order.  Where every face has lowerAddr < upperAddr a sweep is one launch, in which
+ * a row starts as soon as the rows it depends on are done; else the sweeps run
+ * level by level (cells whose faces are independent), one launch per level.
  * Symmetric matrices (it reads upper); no interface entries. */
 #define GIS_PRECOND_DIC 4
 /* OpenFOAM's DILU (diagonal incomplete LU) for asymmetric matrices, from its
  * published algorithm: rD = 1 / (diag - sum over lower faces of
  * upper lower rD_owner) in face order; z = rD r, a forward sweep over the faces
  * with lower, a backward sweep in reverse face order with upper; M^-T exchanges
- * lower and upper.  The same level-scheduled sweeps as DIC.  PBiCG only
+ * lower and upper.  The sweeps run as DIC's do.  PBiCG only
  * (gis_solve_pbicg); gis_solve_pcg rejects it.  No interface entries. */
 #define GIS_PRECOND_DILU 5
 GIS_API int gis_solve_pcg(gis_handle h, int precond, double *x, const double *b,
