@@ -660,6 +660,13 @@ GIS_API int gis_set_late_launches(gis_handle h, int after, int count) {
     return GIS_OK;
 }
 
+GIS_API int gis_set_resident_fault(gis_handle h, int polls) {
+    if (!h) return GIS_ERR_ARG;
+    if (polls < 0) return fail(h, GIS_ERR_ARG, "polls must be >= 0");
+    h->res_fault = polls;
+    return GIS_OK;
+}
+
 GIS_API int gis_set_sweep_polls(gis_handle h, int polls) {
     if (!h) return GIS_ERR_ARG;
     if (polls < 0) return fail(h, GIS_ERR_ARG, "polls must be >= 0");

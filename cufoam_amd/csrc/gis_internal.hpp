@@ -247,6 +247,7 @@ struct gis_context {
     long long res_count[gis::kResCounts] = {};  // gis_get_resident_counts
     int res_skip = 0, res_backoff = 0;          // solves held back after a late grid
     int late_after = 0, late_n = 0;             // gis_set_late_launches (failure-path tests)
+    int res_fault = 0;                          // gis_set_resident_fault (the same)
     int sweep_polls = 0;                        // gis_set_sweep_polls (the same); 0: the default
 
     gis::Schedule sched;

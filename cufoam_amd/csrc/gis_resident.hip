@@ -840,11 +840,13 @@ __global__ __launch_bounds__(kResWG) void k_bicg_res(Mat<double> m, Mat<double> 
     }
 }
 
-// verdict: kResWait, or kResLate for a launch that is to find its grid late
-__global__ void k_res_reset(ResWs ws, KState* st, int verdict) {
+// verdict: kResWait, or kResLate for a launch that is to find its grid late; fault
+// > 0 (gis_set_resident_fault): the waits inside the launch are to run out
+__global__ void k_res_reset(ResWs ws, KState* st, int verdict, int fault) {
     if (threadIdx.x == 0) ws.sync[0] = 0;
     if (threadIdx.x == 1) ws.sync[1] = verdict;
     if (threadIdx.x == 2) st->flag = 0;
+    if (threadIdx.x == 3 && fault > 0) st->slot_fault = fault;
 }
 
 // One waiting grid per GPU in this process: two that share the chip could each
@@ -921,7 +923,7 @@ int run_resident(gis_context* h, int form, Launch&& launch, bool* ran) {
         const ResWs ws{s, reinterpret_cast<int*>(s + n_slot), patience_ticks(h, late)};
         const LateLaunches f = late_launches(h, 1);
         hipLaunchKernelGGL(k_res_reset, dim3(1), dim3(64), 0, h->stream, ws, h->st,
-                           f.first < f.end ? kResLate : kResWait);
+                           f.first < f.end ? kResLate : kResWait, h->res_fault);
         launch(ws);
         GIS_HIP(h, hipGetLastError());
         GIS_TRY(read_state(h));
@@ -939,8 +941,12 @@ int run_resident(gis_context* h, int form, Launch&& launch, bool* ran) {
     }
 }
 
-// 4 words a launch; launches [late0, late1) are to find their grid late
-__global__ void k_res_reset_all(int* sync, int n, int late0, int late1) {
+// 4 words a launch; launches [late0, late1) are to find their grid late; fault as
+// k_res_reset, for the S systems
+__global__ void k_res_reset_all(int* sync, int n, int late0, int late1, KState* st, int S,
+                                int fault) {
+    if (fault > 0)
+        for (int i = threadIdx.x; i < S; i += blockDim.x) st[i].slot_fault = fault;
     for (int i = threadIdx.x; i < 4 * n; i += blockDim.x)
         sync[i] = i % 4 == 1 && i / 4 >= late0 && i / 4 < late1 ? kResLate : 0;
 }
@@ -1081,7 +1087,7 @@ int resident_batch(gis_context* h, const Mat<double>& m, double* r, double* p, d
     for (int late = 0;;) {
         const LateLaunches f = late_launches(h, L);
         hipLaunchKernelGGL(k_res_reset_all, dim3(1), dim3(kWG), 0, h->stream, sync, L, f.first,
-                           f.end);
+                           f.end, B.st.as<KState>(), S, h->res_fault);
         for (int l = 0; l < L; ++l) {
             const ResWs ws{slot, sync + 4 * l, patience_ticks(h, late)};
             const dim3 g((unsigned)(B.res_first[l + 1] - B.res_first[l]));

@@ -111,6 +111,7 @@ SIGNATURES = {
     "gis_set_gamg": (_i, [_vp, _d, _i, _d]),
     "gis_set_slot_fault": (_i, [_vp, _i]),
     "gis_set_late_launches": (_i, [_vp, _i, _i]),
+    "gis_set_resident_fault": (_i, [_vp, _i]),
     "gis_set_sweep_polls": (_i, [_vp, _i]),
     "gis_set_timing_sample": (_i, [_vp, _i]),
     "gis_set_symmetric_storage": (_i, [_vp, _i]),
@@ -613,6 +614,11 @@ class Gis:
         them, find their grid late (gis_set_late_launches)."""
         self._check(self._L.gis_set_late_launches(self._h, int(after), int(count)),
                     "set_late_launches")
+
+    def set_resident_fault(self, polls: int = 0):
+        """Failure-path tests only: the waits inside resident launches give up after
+        `polls` polls (gis_set_resident_fault)."""
+        self._check(self._L.gis_set_resident_fault(self._h, int(polls)), "set_resident_fault")
 
     def set_sweep_polls(self, polls: int = 0):
         """Failure-path tests only: how patient the waits of DIC / DILU sweeps are

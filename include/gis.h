@@ -374,6 +374,10 @@ GIS_API int gis_set_slot_fault(gis_handle h, int polls);
  * `count` of them find their workgroups not all there in time and give up (the
  * kernels exit normally); a launch of one workgroup waits for nobody. */
 GIS_API int gis_set_late_launches(gis_handle h, int after, int count);
+/* Failure-path tests only: gis_set_slot_fault for the reductions and halos inside
+ * resident launches of several workgroups alone (the set-up before them, which
+ * would fail first, works). */
+GIS_API int gis_set_resident_fault(gis_handle h, int polls);
 /* Failure-path tests only: polls in vain after which a waiting wave of a DIC / DILU
  * sweep looks whether the sweep gets on at all (0: the default, 2^20). */
 GIS_API int gis_set_sweep_polls(gis_handle h, int polls);

@@ -322,23 +322,25 @@ def test_late_batch(fresh, use_graph, after, count):
 
 
 def test_two_threads(gpu):
-    """Two handles in two threads: while one's resident solve runs, the other's go
-    stage by stage, with the same bits."""
+    """Two handles in two threads: while one's resident solve runs, a solve of the
+    other goes stage by stage, with the same bits.  Either may come first."""
     import threading
 
     from cufoam_amd.gis import Gis
     s = mesh.laplacian(48, seed=12, shift=1e-3)
     ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, -1.0, 60)
     done = threading.Event()
+    skipped = []
 
     def long_solves():
         with Gis(0) as g:
             g.set_system(s)
             for _ in range(4):
                 g.solve("CG", s.b, s.x0, error=-1.0, max_steps=8000, hist_cap=1)
+            skipped.append(g.resident_counts()["skipped"])
         done.set()
     gpu.set_system(s)
-    before = gpu.resident_counts()
+    before = gpu.resident_counts()["skipped"]
     t = threading.Thread(target=long_solves)
     t.start()
     while not done.is_set():
@@ -346,7 +348,8 @@ def test_two_threads(gpu):
         np.testing.assert_array_equal(hist, ref.hist)
         np.testing.assert_array_equal(x, ref.x)
     t.join()
-    assert gpu.resident_counts()["skipped"] > before["skipped"]
+    skipped.append(gpu.resident_counts()["skipped"] - before)
+    assert len(skipped) == 2 and sum(skipped) > 0
 
 
 @pytest.mark.parametrize("method", ["CG", "BiCG"])
@@ -414,3 +417,55 @@ def test_few_steps_run_as_stages(gpu, edge, method):
                 ref = O.solve(method, A, B[k], np.zeros(s.n_cells), 0.0, steps)
                 assert it[k] == ref.iterations and nf[k] == ref.hist[-1]
                 np.testing.assert_array_equal(X[k], ref.x)
+
+
+@pytest.mark.parametrize("method", ["CG", "BiCG"])
+@pytest.mark.parametrize("edge", [14, 66])
+def test_failed_launch_is_reported_and_recovers(fresh, method, edge):
+    """The bounded waits inside a launch, forced from the host: every workgroup gives
+    up after 4 polls and exits, the solve reports GIS_ERR_SYNC, and the next one has
+    its bits again.  66^3: two tiles a workgroup (CG)."""
+    from cufoam_amd.gis import GisError
+    s = mesh.laplacian(edge, seed=15, shift=0.1, symmetric=method == "CG")
+    if method == "BiCG" and edge == 66:
+        s = mesh.laplacian(63, seed=15, shift=0.1, symmetric=False)
+    fresh.set_system(s)
+    A = O.ldu2csr(s)
+    ref = O.solve(method, A, s.b, s.x0, 0.0, 40)
+    B = np.stack([s.b, s.b[::-1]])
+    fresh.set_resident_fault(4)
+    for call in (lambda g: g.solve(method, s.b, s.x0, error=0.0, max_steps=40),
+                 lambda g: g.solve_multi(method, B, None, error=0.0, max_steps=40)):
+        with pytest.raises(GisError) as e:
+            call(fresh)
+        assert e.value.status == 13
+    fresh.set_resident_fault(0)
+    (x, hist, _), grew = counted(
+        fresh, lambda g: g.solve(method, s.b, s.x0, error=0.0, max_steps=40))
+    assert grew == {"ran": 1}
+    np.testing.assert_array_equal(hist, ref.hist)
+    np.testing.assert_array_equal(x, ref.x)
+    X, it, nf, st = fresh.solve_multi(method, B, None, error=0.0, max_steps=40)
+    np.testing.assert_array_equal(X[0], ref.x)
+
+
+def test_failed_batch_launch_is_reported_and_recovers(fresh):
+    """The same in a batch: systems of several workgroups fail, one of a single
+    workgroup waits for nobody; then every system has its bits again."""
+    from cufoam_amd.gis import GisError
+    systems = [mesh.laplacian(n, seed=70 + i, shift=1e-2) for i, n in enumerate([14, 9, 40])]
+    b = np.concatenate([s.b for s in systems])
+    fresh.batch_set_systems(systems)
+    fresh.set_resident_fault(4)
+    with pytest.raises(GisError) as e:
+        fresh.batch_solve(b, None, 1e-8, 300)
+    assert e.value.status == 13
+    fresh.set_resident_fault(0)
+    (x, it, nf, st), grew = counted(fresh, lambda g: g.batch_solve(b, None, 1e-8, 300))
+    assert set(grew) == {"ran"}
+    off = 0
+    for i, s in enumerate(systems):
+        ref = O.solve("CG", O.ldu2csr(s), s.b, s.x0, 1e-8, 300)
+        assert it[i] == ref.iterations and nf[i] == ref.hist[-1]
+        np.testing.assert_array_equal(x[off:off + s.n_cells], ref.x)
+        off += s.n_cells
